@@ -72,6 +72,28 @@ def test_row_stats_bit_exact(device, oracle, vocab):
         assert np.float32(z[r]).view(np.uint32) == np.float32(oz).view(np.uint32), (r, z[r], oz)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("vocab,start,stride", [
+    (1, 1, 3), (5, 0, 5), (2047, 0, 2047), (2048, 1, 2049), (2050, 3, 2055), (4098, 2, 4100),
+    (16384, 1, 16387), (16385, 0, 16385), (18433, 1, 18435), (32770, 0, 32771)])
+def test_row_stats_unaligned_rows_bit_exact(device, oracle, dtype, vocab, start, stride):
+    """Rows whose start, stride or length is no multiple of four elements:
+    one slab or less, whole slabs only, a partial last slab on the first and
+    on another wave, one and two rounds of slabs a wave."""
+    rng = np.random.default_rng(vocab + start)
+    flat = torch.from_numpy((rng.standard_normal(5 * stride + start) * 4).astype(np.float32))
+    flat = flat.to(dtype)
+    flat[start + stride::9] = -torch.inf
+    rows = flat.to(device)[start:start + 5 * stride].view(5, stride)[:, :vocab]
+    m, z = ops.row_stats(rows)
+    m, z = m.cpu().numpy(), z.cpu().numpy()
+    host = flat.float().numpy()[start:start + 5 * stride].reshape(5, stride)[:, :vocab]
+    for r in range(5):
+        om, oz = oracle.row_stats(np.ascontiguousarray(host[r]))
+        assert m[r] == om
+        assert np.float32(z[r]).view(np.uint32) == np.float32(oz).view(np.uint32), (r, z[r], oz)
+
+
 @pytest.mark.parametrize("seed", [0, 1, 2, 3])
 def test_tiny_vocab_trees_bit_exact(device, oracle, seed):
     case = tree_problem(seed, num_requests=6, nodes=[16, 1, 9, 16, 3, 12], vocab=4096)
