@@ -543,10 +543,10 @@ __global__ __launch_bounds__(kLmThreads, RowTile<R>::kBlocksPerCU) void lm_head_
   lm_tile<R, kPacked, false>(a, smem, vt, rt, 0);
 }
 
-// Ping-pong form of the 256-row tile (more than 128 projected rows): eight
-// waves, two per SIMD, in two groups (waves 0-3 and 4-7) half a stage apart.
-// Wave w owns tokens [128*(w&1), +128) and rows [64*(2*(w>>2) + ((w>>1)&1)),
-// +64) of the 256 x 256 tile: 8 x 4 blocks of 16 x 16, 128 accumulators.  In
+// Ping-pong form (more than 128 projected rows): eight waves, two per SIMD, in
+// two groups (waves 0-3 and 4-7) half a stage apart.  Wave w owns tokens
+// [128*(w&1), +128) and the 16 NB rows 16 NB (2*(w>>2) + ((w>>1)&1)) .. of a
+// 256-token x 64 NB-row tile: 8 x NB blocks of 16 x 16, 32 NB accumulators.  In
 // phase 2t group A (waves 0-3) reads stage t's fragments from LDS and issues
 // its share of the copies of stage t+3 while group B multiplies stage t-1; in
 // phase 2t+1 the groups swap roles.  The two waves of a SIMD thus alternate
@@ -556,38 +556,59 @@ __global__ __launch_bounds__(kLmThreads, RowTile<R>::kBlocksPerCU) void lm_head_
 // products, their order per accumulator (ascending hidden dims) and the
 // epilogue's statistics order are those of lm_head_kernel, so the logits and
 // statistics are bit-identical.
+//
+// Row tiles: the rows' 64-row units are spread evenly over the fewest tiles of
+// at most kPpMaxUnits units (row_tile below), so that a call multiplies at
+// most 63 empty rows.  A phase's MFMAs take 128 NB cycles beside 48 NB + 320
+// cycles of LDS traffic (the other group's fragment reads and the copies), so
+// a larger NB also spends fewer LDS cycles per product.
 constexpr int kPpThreads = 512;
+constexpr int kPpMaxUnits = 5;
+template <int NB>
 struct PpTile {
-  static constexpr int kRows = 256;
-  static constexpr int kXBytes = kRows * kStepK * 2;  // hidden bytes per stage (16 KiB)
-  static constexpr int kStage = kWBytes + kXBytes;     // 32 KiB
-  static constexpr int kDmas = 4;                      // copies per wave per stage
-  static constexpr int kStaging = 8 * 64 * kOutPitch;  // 64 rows x 128 tokens per wave
-  static constexpr int kLds = kLmStages * kStage > kStaging ? kLmStages * kStage : kStaging;
+  static constexpr int kRows = 64 * NB;
+  static constexpr int kWaveRows = 16 * NB;
+  static constexpr int kXBytes = kRows * kStepK * 2;  // hidden bytes per stage
+  static constexpr int kStage = kWBytes + kXBytes;
+  // Hidden copies (16 rows each) per stage of a wave of group G.
+  template <int G>
+  static constexpr int kXCopies = G == 0 ? (NB + 1) / 2 : NB / 2;
+  template <int G>
+  static constexpr int kDmas = 2 + kXCopies<G>;
 };
+constexpr int kPpStaging = 8 * 2 * 16 * kOutPitch;  // two 16-row blocks per wave
+constexpr int kPpLds = kLmStages * PpTile<kPpMaxUnits>::kStage;
+static_assert(kPpStaging <= kPpLds, "the output staging reuses the ring");
 
-template <bool kPacked>
-__global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs a, int v_tiles,
-                                                                    int r_tiles) {
-  using T = PpTile;
-  __shared__ __align__(1024) unsigned char smem[T::kLds];
-  int vt, rt;
-  if (!tile_of(blockIdx.x, v_tiles, r_tiles, vt, rt)) return;
+// Row tile rt of r_tiles over `units` 64-row units: its first row and units.
+__device__ __forceinline__ void row_tile(int units, int r_tiles, int rt, int& r0, int& nb) {
+  const int base = units / r_tiles;
+  const int extra = units - base * r_tiles;  // the first `extra` tiles take one more
+  nb = base + (rt < extra ? 1 : 0);
+  r0 = 64 * (base * rt + min(rt, extra));
+}
+
+template <bool kPacked, int NB>
+__device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* smem, int vt,
+                                        int r0) {
+  using T = PpTile<NB>;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2;               // 0: group A, 1: group B
   const int wv = wave & 1;                 // 128-token half of the tile
-  const int wr = 2 * grp + ((wave >> 1) & 1);  // 64-row quarter of the tile
+  const int wr = 2 * grp + ((wave >> 1) & 1);  // 16 NB-row quarter of the tile
   const int g = lane >> 4;
   const int V = a.vocab;
   const int v0 = vt * kTileV;
-  const int r0 = rt * T::kRows;
 
   // Copy slots, with the operand stage layout of lm_head_kernel: weight copy q
   // (rows 16q .. 16q+15, 64 bytes each) at LDS 1024 q, hidden copy q at
-  // kWBytes + 1024 q; wave w issues weight and hidden copies 2w and 2w+1.
-  uint32_t w_off[2], w_lds[2], x_off[2], x_lds[2];
+  // kWBytes + 1024 q; wave w issues weight copies 2w and 2w+1, and the waves
+  // of group A hidden copies w, w+4, .., those of group B the copies after
+  // group A's in the same way.
+  constexpr int kXa = T::template kXCopies<0>;
+  uint32_t w_off[2], w_lds[2], x_off[kXa], x_lds[kXa];
   const int steps = a.hidden_size / kStepK;
   const unsigned char* wbase =
       static_cast<const unsigned char*>(a.weight_dev) +
@@ -597,16 +618,23 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
   const unsigned char* xbase = static_cast<const unsigned char*>(a.hidden_dev);
   bool bad_index = false;
   const int g_lane = (lane & 3) ^ ((lane >> 3) & 3);  // swz(row) = (row >> 1) & 3
+  const int dim = 8 * g_lane;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int q = 2 * wave + i;
     const int row = 16 * q + (lane >> 2);
-    const int dim = 8 * g_lane;
     const int tok = min(v0 + row, V - 1) - v0;
     w_off[i] = kPacked ? static_cast<uint32_t>(row * kStepK * 2 + dim * 2)
                        : static_cast<uint32_t>((static_cast<int64_t>(tok) * a.weight_row_stride +
                                                 dim) * 2);
     w_lds[i] = static_cast<uint32_t>(1024 * q);
+  }
+#pragma unroll
+  for (int i = 0; i < kXa; ++i) {
+    // Group B's last copy slot is unused when NB is odd; its index stays
+    // inside the tile.
+    const int q = min(4 * (grp == 0 ? i : kXa + i) + (wave & 3), 4 * NB - 1);
+    const int row = 16 * q + (lane >> 2);
     const int prow = min(r0 + row, a.num_rows - 1);
     int src = a.row_index_dev != nullptr ? a.row_index_dev[prow] : prow;
     if (src < 0 || src >= a.num_hidden_rows) {
@@ -619,39 +647,16 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
   if (bad_index && a.status_dev != nullptr) atomicExch(a.status_dev, SG_EINVAL);
 
   const uint32_t ring = lds_addr(smem);
-  auto issue = [&](int t) {
-    const uint32_t stage = ring + (t % kLmStages) * T::kStage;
-    const unsigned char* wk = wbase + static_cast<int64_t>(t) * kWStep;
-    const unsigned char* xk = xbase + static_cast<int64_t>(t) * kStepK * 2;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(wk, w_off[i], stage + w_lds[i]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(xk, x_off[i], stage + x_lds[i]);
-  };
-
   // Fragments as in lm_head_kernel: lane l reads row l%16 of a 16-row block,
   // chunk l/16, at LDS chunk (l/16) ^ swz(l%16).
   const int lq = (lane & 15) * 64 + 16 * (g ^ (((lane & 15) >> 1) & 3));
-  const int a_base = wv * 8 * 1024;      // this wave's 128 token rows
-  const int b_base = kWBytes + wr * 4 * 1024;  // this wave's 64 hidden rows
-  // Waits until at most `newer` stages of this wave's copies are in flight.
-  auto wait_newer = [&](int newer) {
-    if (newer >= 2) {
-      __builtin_amdgcn_s_waitcnt(vmcnt_encoding(2 * T::kDmas));
-    } else if (newer == 1) {
-      __builtin_amdgcn_s_waitcnt(vmcnt_encoding(T::kDmas));
-    } else {
-      __builtin_amdgcn_s_waitcnt(vmcnt_encoding(0));
-    }
-  };
-  for (int t = 0; t < kLmStages - 1 && t < steps; ++t) issue(t);
-  wait_newer(min(kLmStages - 2, steps - 1));  // stage 0 has landed
-  __syncthreads();
+  const int a_base = wv * 8 * 1024;                // this wave's 128 token rows
+  const int b_base = kWBytes + wr * NB * 1024;     // this wave's hidden rows
 
   // The main loop and the epilogue, once per group (G known at compile time,
   // so each copy is straight-line code: no branch chooses between product
   // sites, which would make the compiler copy the accumulators).  A barrier
-  // counts arrivals, not instructions: both copies pass 2 steps + 1 barriers.
+  // counts arrivals, not instructions: both copies pass 2 steps + 2 barriers.
   // Group A: phase 2t reads stage t and issues stage t+3, phase 2t+1
   // multiplies.  Group B: one idle phase, then phase 2t+1 reads stage t and
   // issues stage t+3, phase 2t+2 multiplies.  Before the barrier that ends
@@ -659,28 +664,38 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
   // p+1, so that the barrier publishes the whole stage.
   auto body = [&](auto group) {
     constexpr int G = decltype(group)::value;
+    constexpr int kDmas = T::template kDmas<G>;
+    auto issue = [&](int t) {
+      const uint32_t stage = ring + (t % kLmStages) * T::kStage;
+      const unsigned char* wk = wbase + static_cast<int64_t>(t) * kWStep;
+      const unsigned char* xk = xbase + static_cast<int64_t>(t) * kStepK * 2;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) dma16(wk, w_off[i], stage + w_lds[i]);
+#pragma unroll
+      for (int i = 0; i < T::template kXCopies<G>; ++i) dma16(xk, x_off[i], stage + x_lds[i]);
+    };
     // acc[tb][rb][i]: token 16 tb + 4 g + i of this wave's 128, row
-    // 16 rb + n of its 64 (lm_head_kernel's products and order).
-    floatx4 acc[8][4];
+    // 16 rb + n of its 16 NB (lm_head_kernel's products and order).
+    floatx4 acc[8][NB];
 #pragma unroll
     for (int tb = 0; tb < 8; ++tb)
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb) acc[tb][rb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    bf16x8 fa[8], fb[4];
+      for (int rb = 0; rb < NB; ++rb) acc[tb][rb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 fa[8], fb[NB];
     auto read_frags = [&](int t) {
       const unsigned char* st = smem + (t % kLmStages) * T::kStage;
 #pragma unroll
       for (int tb = 0; tb < 8; ++tb)
         fa[tb] = as_bf16x8(*reinterpret_cast<const uint4*>(st + a_base + tb * 1024 + lq));
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < NB; ++rb)
         fb[rb] = as_bf16x8(*reinterpret_cast<const uint4*>(st + b_base + rb * 1024 + lq));
     };
     auto mma = [&]() {
 #pragma unroll
       for (int tb = 0; tb < 8; ++tb)
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
+        for (int rb = 0; rb < NB; ++rb)
           acc[tb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[tb], fb[rb], acc[tb][rb], 0, 0,
                                                                 0);
     };
@@ -691,13 +706,7 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
     auto stage_step = [&](int t, auto newer) {
       constexpr int N = decltype(newer)::value;
       auto wait_next = [&]() {
-        if constexpr (N >= 2) {
-          __builtin_amdgcn_s_waitcnt(vmcnt_encoding(2 * T::kDmas));
-        } else if constexpr (N == 1) {
-          __builtin_amdgcn_s_waitcnt(vmcnt_encoding(T::kDmas));
-        } else if constexpr (N == 0) {
-          __builtin_amdgcn_s_waitcnt(vmcnt_encoding(0));
-        }
+        if constexpr (N >= 0) __builtin_amdgcn_s_waitcnt(vmcnt_encoding(N * kDmas));
       };
       read_frags(t);
       if constexpr (N >= 2) issue(t + kLmStages - 1);
@@ -718,9 +727,14 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
       __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
     };
-    static_assert(kLmStages == 4, "the tail below is written for a four-stage ring");
+    static_assert(kLmStages == 4, "the prologue and the tail are written for a four-stage ring");
+    // steps >= 3 (the launcher's condition): three stages issued ahead, stage
+    // 0 landed when two of them may still be in flight.
+    for (int t = 0; t < kLmStages - 1; ++t) issue(t);
+    __builtin_amdgcn_s_waitcnt(vmcnt_encoding(2 * kDmas));
+    __syncthreads();
     if constexpr (G == 1) __syncthreads();  // phase 0: group A reads stage 0
-    // steps >= 3 (the launcher's condition); stage t+3 exists for t < steps-3.
+    // Stage t+3 exists for t < steps-3.
     for (int t = 0; t + kLmStages - 1 < steps; ++t) stage_step(t, std::integral_constant<int, 2>{});
     stage_step(steps - 3, std::integral_constant<int, 1>{});
     stage_step(steps - 2, std::integral_constant<int, 0>{});
@@ -729,24 +743,50 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
     // The ring is free (every barrier above waited for the LDS reads): it
     // becomes the output staging area.
 
-    // Epilogue (lm_head_kernel's, for the wave's four 16-row blocks).
+    // Epilogue (lm_head_kernel's), one 16-row block at a time: statistics and
+    // staging, then the block's rows written as whole 256-byte segments (four
+    // rows an instruction).  Consecutive blocks alternate between two staging
+    // buffers of the wave.
     const int tok0 = v0 + 128 * wv;
     const bool tile_live = tok0 < V;
     const int n_tiles = (V + kStatTokens - 1) / kStatTokens;
-    unsigned char* stage = smem + wave * 64 * kOutPitch;
+    unsigned char* stage = smem + wave * 2 * 16 * kOutPitch;
+    uint16_t* out = static_cast<uint16_t*>(a.logits_dev);
     auto epilogue = [&](auto full) {
+      constexpr bool kFull = decltype(full)::value;
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb) {
-        const int row_local = 16 * rb + (lane & 15);
-        const int row = r0 + 64 * wr + row_local;
-        const float2 mz = block_epilogue<decltype(full)::value>(acc, rb, tok0, V, g,
-                                                                stage + row_local * kOutPitch);
+      for (int rb = 0; rb < NB; ++rb) {
+        unsigned char* buf = stage + (rb & 1) * 16 * kOutPitch;
+        const int row0 = r0 + T::kWaveRows * wr + 16 * rb;  // the block's first projected row
+        const int row = row0 + (lane & 15);
+        const float2 mz =
+            block_epilogue<kFull>(acc, rb, tok0, V, g, buf + (lane & 15) * kOutPitch);
         if (g == 0 && tile_live && row < a.num_rows) {
           float* dst =
               a.tile_stats_dev + (static_cast<int64_t>(row) * n_tiles + tok0 / kStatTokens) * 2;
           *reinterpret_cast<float2*>(dst) = mz;
         }
-        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_wave_barrier();
+        const int chunk = lane & 15;
+        const int tok = tok0 + 8 * chunk;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int out_row = row0 + 4 * i + (lane >> 4);
+          const uint4 v = *reinterpret_cast<const uint4*>(buf + (4 * i + (lane >> 4)) * kOutPitch +
+                                                          16 * chunk);
+          if (out_row >= a.num_rows || (!kFull && tok >= V)) continue;
+          uint16_t* dst = out + static_cast<int64_t>(out_row) * a.logits_row_stride + tok;
+          if (kFull || tok + 8 <= V) {
+            *reinterpret_cast<uint4*>(dst) = v;
+          } else {
+            for (int e = 0; tok + e < V; ++e) {
+              const uint32_t w =
+                  (e >> 1) == 0 ? v.x : (e >> 1) == 1 ? v.y : (e >> 1) == 2 ? v.z : v.w;
+              dst[e] = static_cast<uint16_t>((e & 1) ? (w >> 16) : (w & 0xffffu));
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one 16-row block at a time (registers)
       }
     };
     if (tok0 + kStatTokens <= V) {
@@ -754,32 +794,39 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
     } else {
       epilogue(std::false_type{});
     }
-    __builtin_amdgcn_wave_barrier();
-    if (!tile_live) return;
-    uint16_t* out = static_cast<uint16_t*>(a.logits_dev);
-#pragma unroll 4
-    for (int i = 0; i < 16; ++i) {
-      const int row_local = 4 * i + (lane >> 4);
-      const int row = r0 + 64 * wr + row_local;
-      const int chunk = lane & 15;
-      const int tok = tok0 + 8 * chunk;
-      const uint4 v = *reinterpret_cast<const uint4*>(stage + row_local * kOutPitch + 16 * chunk);
-      if (row >= a.num_rows || tok >= V) continue;
-      uint16_t* dst = out + static_cast<int64_t>(row) * a.logits_row_stride + tok;
-      if (tok + 8 <= V) {
-        *reinterpret_cast<uint4*>(dst) = v;
-      } else {
-        for (int e = 0; tok + e < V; ++e) {
-          const uint32_t w = (e >> 1) == 0 ? v.x : (e >> 1) == 1 ? v.y : (e >> 1) == 2 ? v.z : v.w;
-          dst[e] = static_cast<uint16_t>((e & 1) ? (w >> 16) : (w & 0xffffu));
-        }
-      }
-    }
   };
   if (grp == 0) {
     body(std::integral_constant<int, 0>{});
   } else {
     body(std::integral_constant<int, 1>{});
+  }
+}
+
+// Workgroup b -> (vocabulary tile, row tile).  The row tiles of one vocabulary
+// tile take consecutive slots of one XCD (tile_of); the last vocabulary tiles,
+// fewer than one per XCD, go round the XCDs one row tile at a time, so that no
+// XCD has more than one workgroup more than another.
+template <bool kPacked>
+__global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs a, int v_tiles,
+                                                                    int r_tiles, int units) {
+  __shared__ __align__(1024) unsigned char smem[kPpLds];
+  const int b = static_cast<int>(blockIdx.x);
+  const int v_even = v_tiles / kLmXcds * kLmXcds;
+  int vt, rt;
+  if (b < v_even * r_tiles) {
+    tile_of(b, v_even, r_tiles, vt, rt);
+  } else {
+    const int i = b - v_even * r_tiles;
+    vt = v_even + i / r_tiles;
+    rt = i % r_tiles;
+  }
+  int r0, nb;
+  row_tile(units, r_tiles, rt, r0, nb);
+  switch (nb) {
+    case 5: pp_tile<kPacked, 5>(a, smem, vt, r0); break;
+    case 4: pp_tile<kPacked, 4>(a, smem, vt, r0); break;
+    case 3: pp_tile<kPacked, 3>(a, smem, vt, r0); break;
+    default: pp_tile<kPacked, 2>(a, smem, vt, r0); break;
   }
 }
 
@@ -894,16 +941,16 @@ int launch_lm_head(const SgLmHeadArgs& a, bool packed, hipStream_t s) {
     return SG_OK;
   };
   auto launch_pp = [&]() -> int {
-    const int r_tiles = (a.num_rows + PpTile::kRows - 1) / PpTile::kRows;
-    const int64_t blocks =
-        static_cast<int64_t>((v_tiles + kLmXcds - 1) / kLmXcds) * kLmXcds * r_tiles;
+    const int units = (a.num_rows + 63) / 64;  // >= 3: every tile has two units or more
+    const int r_tiles = (units + kPpMaxUnits - 1) / kPpMaxUnits;
+    const int64_t blocks = static_cast<int64_t>(v_tiles) * r_tiles;
     SG_REQUIRE(blocks < INT32_MAX, "wave too large");
     if (packed) {
       lm_head_pp_kernel<true><<<dim3(static_cast<unsigned>(blocks)), dim3(kPpThreads), 0, s>>>(
-          a, v_tiles, r_tiles);
+          a, v_tiles, r_tiles, units);
     } else {
       lm_head_pp_kernel<false><<<dim3(static_cast<unsigned>(blocks)), dim3(kPpThreads), 0, s>>>(
-          a, v_tiles, r_tiles);
+          a, v_tiles, r_tiles, units);
     }
     SG_LAUNCH_CHECK();
     return SG_OK;
