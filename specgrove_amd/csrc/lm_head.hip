@@ -174,72 +174,90 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
 
-// Epilogue of one 16-row block of a wave's 128-token statistics tile.  Lane
-// (g, n) = (lane / 16, lane % 16) holds in acc[tb][rb][i] row n of the block
-// at token tok0 + 16 tb + 4 g + i (the 16x16 MFMA output layout).  Rounds
-// them to bf16, writes the bf16 logits into the lane's staging row (128
-// tokens) and returns the tile's (m, z) of the statistics contract: m the
-// maximum (every lane), z = z_0 + z_1 (lanes g < 2) with z_h the sum of
-// E(x - m) over the half's tokens (bit 2 of the token = h) in increasing
-// token order.  A half's tokens alternate between lanes g = h and g = h + 2
-// in runs of four, so the lower lanes take the upper lanes' values and add
-// them in that order.  kFull: every token of the tile is below V, so no
+// Epilogue of one or two 16-row blocks (rb, rb + 1) of a wave's 128-token
+// statistics tile.  Lane (g, n) = (lane / 16, lane % 16) holds in acc[tb][rb][i]
+// row n of block rb at token tok0 + 16 tb + 4 g + i (the 16x16 MFMA output
+// layout).  Rounds them to bf16, writes the bf16 logits into the lane's staging
+// rows (128 tokens; the second block's `pitch2` bytes after the first's) and
+// returns the tile's (m, z) of the statistics contract, in lanes g = 0 those of
+// row n of block rb and in lanes g = 2 those of row n of block rb + 1: m the
+// maximum, z = z_0 + z_1 with z_h the sum of E(x - m) over the half's tokens
+// (bit 2 of the token = h) in increasing token order.  A half's tokens
+// alternate between lanes g = h and g = h + 2 in runs of four.  One
+// permlane32_swap of a block's values with the other block's gives the lower
+// lanes both runs of the first block and the upper lanes both of the second, so
+// every lane adds values that count; a lone block's lower lanes take the upper
+// lanes' values.  (The epilogue is bound by its VALU instructions, 698 a block
+// alone; in pairs a call of 256 rows, H 512, V 151,936 took 81.5 us, before 88;
+// 784 rows, H 4096: 866, before 875.)  kFull: every token of the tile is below V, so no
 // token needs a mask (the masks are 64-bit lane masks per token, and 32 of
 // them do not fit the scalar registers).
-template <bool kFull, int NB>
+template <bool kFull, int B, int NB>
 __device__ __forceinline__ float2 block_epilogue(const floatx4 (&acc)[8][NB], int rb, int tok0,
-                                                 int V, int g, unsigned char* stage_row) {
-  float x[32];
-#pragma unroll
-  for (int tb = 0; tb < 8; ++tb)
-#pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-      const uint32_t pr = cvt_pk_bf16(acc[tb][rb][i], acc[tb][rb][i + 1]);
-      x[4 * tb + i] = __uint_as_float(pr << 16);
-      x[4 * tb + i + 1] = __uint_as_float(pr & 0xffff0000u);
-    }
+                                                 int V, int g, unsigned char* stage_row,
+                                                 int pitch2) {
+  static_assert(B == 1 || B == 2, "one block or a pair");
   auto live = [&](int tb, int i) { return kFull || tok0 + 16 * tb + 4 * g + i < V; };
-  float m = -__builtin_inff();
+  float x[B][32], m[B], mc[B];
 #pragma unroll
-  for (int tb = 0; tb < 8; ++tb)
+  for (int b = 0; b < B; ++b) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m = live(tb, i) ? fmaxf(m, x[4 * tb + i]) : m;
-  m = fmaxf(m, __shfl_xor(m, 16));
-  m = half_max(m);
-  // Tokens at or past V add exactly 0 (z stays a non-negative sum).
-  const float mc = (m == -__builtin_inff()) ? 0.0f : m;
+    for (int tb = 0; tb < 8; ++tb)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        const uint32_t pr = cvt_pk_bf16(acc[tb][rb + b][i], acc[tb][rb + b][i + 1]);
+        x[b][4 * tb + i] = __uint_as_float(pr << 16);
+        x[b][4 * tb + i + 1] = __uint_as_float(pr & 0xffff0000u);
+      }
+    float v = -__builtin_inff();
+#pragma unroll
+    for (int tb = 0; tb < 8; ++tb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v = live(tb, i) ? fmaxf(v, x[b][4 * tb + i]) : v;
+    v = fmaxf(v, __shfl_xor(v, 16));
+    m[b] = half_max(v);
+    // Tokens at or past V add exactly 0 (z stays a non-negative sum).
+    mc[b] = (m[b] == -__builtin_inff()) ? 0.0f : m[b];
+  }
   float z = 0.0f;
 #pragma unroll
   for (int tb = 0; tb < 8; ++tb) {
-    float e[4], pe[4];
+    float lo[4], hi[4];  // the runs of lanes g and g + 2 (g < 2) of this lane's block
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float v = sg_exp_nonpos(x[4 * tb + i] - mc);
-      e[i] = live(tb, i) ? v : 0.0f;
+      float e[B];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const float v = sg_exp_nonpos(x[b][4 * tb + i] - mc[b]);
+        e[b] = live(tb, i) ? v : 0.0f;
+      }
+      // r[0] = lower lanes of e[0] | lower lanes of e[B-1],
+      // r[1] = upper lanes of e[0] | upper lanes of e[B-1].
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(e[0]),
+                                                      __float_as_uint(e[B - 1]), false, false);
+      lo[i] = __uint_as_float(r[0]);
+      hi[i] = __uint_as_float(r[1]);
     }
-    // Lanes 0..31 receive lanes 32..63's values (the same tokens + 8).
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(e[i]),
-                                                      __float_as_uint(e[i]), false, false);
-      pe[i] = __uint_as_float(r[1]);
-    }
+    for (int i = 0; i < 4; ++i) z = z + lo[i];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) z = z + e[i];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) z = z + pe[i];
+    for (int i = 0; i < 4; ++i) z = z + hi[i];
   }
-  z = z + __shfl_xor(z, 16);  // z_0 + z_1 in lanes g = 0 and g = 1
-  // bf16 logits into the staging row (LDS rows of 128 tokens); x is already
+  z = z + __shfl_xor(z, 16);  // z_0 + z_1
+  // bf16 logits into the staging rows (LDS rows of 128 tokens); x is already
   // bf16, so packing keeps its upper halves.
-  auto pack = [&](int i) {
-    return __builtin_amdgcn_perm(__float_as_uint(x[i + 1]), __float_as_uint(x[i]), 0x07060302u);
-  };
 #pragma unroll
-  for (int tb = 0; tb < 8; ++tb)
-    *reinterpret_cast<uint2*>(stage_row + 2 * (16 * tb + 4 * g)) =
-        make_uint2(pack(4 * tb), pack(4 * tb + 2));
-  return make_float2(m, z);
+  for (int b = 0; b < B; ++b) {
+    auto pack = [&](int i) {
+      return __builtin_amdgcn_perm(__float_as_uint(x[b][i + 1]), __float_as_uint(x[b][i]),
+                                   0x07060302u);
+    };
+#pragma unroll
+    for (int tb = 0; tb < 8; ++tb)
+      *reinterpret_cast<uint2*>(stage_row + b * pitch2 + 2 * (16 * tb + 4 * g)) =
+          make_uint2(pack(4 * tb), pack(4 * tb + 2));
+  }
+  return make_float2(B == 2 && g >= 2 ? m[B - 1] : m[0], z);
 }
 
 // Workgroup b -> (vocabulary tile, row tile): the dispatcher places b on XCD
@@ -470,24 +488,26 @@ __device__ __forceinline__ void lm_tile(const SgLmHeadArgs& a, unsigned char* sm
   mma(f1);
   __syncthreads();  // the ring is free: it becomes the output staging area
 
-  // Epilogue, one 16-row block at a time.
+  // Epilogue, two 16-row blocks at a time.
   const int tok0 = v0 + 128 * wv;           // first token of this wave's statistics tile
   const bool tile_live = tok0 < V;
   const int n_tiles = (V + kStatTokens - 1) / kStatTokens;
   unsigned char* stage = smem + wave * T::kWaveRows * kOutPitch;
   auto epilogue = [&](auto full) {
+    constexpr int B = NB >= 2 ? 2 : 1;
 #pragma unroll
-    for (int rb = 0; rb < NB; ++rb) {
-      const int row_local = 16 * rb + (lane & 15);          // row inside this wave's rows
-      const int row = r0 + T::kWaveRows * wr + row_local;  // projected row
-      const float2 mz = block_epilogue<decltype(full)::value>(acc, rb, tok0, V, g,
-                                                              stage + row_local * kOutPitch);
-      if (g == 0 && tile_live && row < a.num_rows) {
+    for (int rb = 0; rb < NB; rb += B) {
+      const int row_local = 16 * rb + (lane & 15);  // row inside this wave's rows
+      const float2 mz = block_epilogue<decltype(full)::value, B>(
+          acc, rb, tok0, V, g, stage + row_local * kOutPitch, 16 * kOutPitch);
+      // Lanes g = 0: block rb, g = 2: block rb + 1.
+      const int row = r0 + T::kWaveRows * wr + row_local + 8 * g;  // projected row
+      if ((g == 0 || (B == 2 && g == 2)) && tile_live && row < a.num_rows) {
         float* dst =
             a.tile_stats_dev + (static_cast<int64_t>(row) * n_tiles + tok0 / kStatTokens) * 2;
         *reinterpret_cast<float2*>(dst) = mz;
       }
-      __builtin_amdgcn_sched_barrier(0);  // one 16-row block at a time (registers)
+      __builtin_amdgcn_sched_barrier(0);  // one pair of blocks at a time (registers)
     }
   };
   if (tok0 + kStatTokens <= V) {
@@ -743,10 +763,9 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
     // The ring is free (every barrier above waited for the LDS reads): it
     // becomes the output staging area.
 
-    // Epilogue (lm_head_kernel's), one 16-row block at a time: statistics and
-    // staging, then the block's rows written as whole 256-byte segments (four
-    // rows an instruction).  Consecutive blocks alternate between two staging
-    // buffers of the wave.
+    // Epilogue (lm_head_kernel's), two 16-row blocks at a time: statistics and
+    // staging, then the blocks' rows written as whole 256-byte segments (four
+    // rows an instruction).
     const int tok0 = v0 + 128 * wv;
     const bool tile_live = tok0 < V;
     const int n_tiles = (V + kStatTokens - 1) / kStatTokens;
@@ -754,14 +773,13 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
     uint16_t* out = static_cast<uint16_t*>(a.logits_dev);
     auto epilogue = [&](auto full) {
       constexpr bool kFull = decltype(full)::value;
-#pragma unroll
-      for (int rb = 0; rb < NB; ++rb) {
-        unsigned char* buf = stage + (rb & 1) * 16 * kOutPitch;
-        const int row0 = r0 + T::kWaveRows * wr + 16 * rb;  // the block's first projected row
-        const int row = row0 + (lane & 15);
-        const float2 mz =
-            block_epilogue<kFull>(acc, rb, tok0, V, g, buf + (lane & 15) * kOutPitch);
-        if (g == 0 && tile_live && row < a.num_rows) {
+      auto blocks = [&](int rb, auto count) {
+        constexpr int B = decltype(count)::value;
+        const int row0 = r0 + T::kWaveRows * wr + 16 * rb;  // the blocks' first projected row
+        const float2 mz = block_epilogue<kFull, B>(
+            acc, rb, tok0, V, g, stage + (lane & 15) * kOutPitch, 16 * kOutPitch);
+        const int row = row0 + (lane & 15) + 8 * g;  // lanes g = 0: block rb, g = 2: rb + 1
+        if ((g == 0 || (B == 2 && g == 2)) && tile_live && row < a.num_rows) {
           float* dst =
               a.tile_stats_dev + (static_cast<int64_t>(row) * n_tiles + tok0 / kStatTokens) * 2;
           *reinterpret_cast<float2*>(dst) = mz;
@@ -770,10 +788,10 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
         const int chunk = lane & 15;
         const int tok = tok0 + 8 * chunk;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4 * B; ++i) {
           const int out_row = row0 + 4 * i + (lane >> 4);
-          const uint4 v = *reinterpret_cast<const uint4*>(buf + (4 * i + (lane >> 4)) * kOutPitch +
-                                                          16 * chunk);
+          const uint4 v = *reinterpret_cast<const uint4*>(
+              stage + (4 * i + (lane >> 4)) * kOutPitch + 16 * chunk);
           if (out_row >= a.num_rows || (!kFull && tok >= V)) continue;
           uint16_t* dst = out + static_cast<int64_t>(out_row) * a.logits_row_stride + tok;
           if (kFull || tok + 8 <= V) {
@@ -786,8 +804,11 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
             }
           }
         }
-        __builtin_amdgcn_sched_barrier(0);  // one 16-row block at a time (registers)
-      }
+        __builtin_amdgcn_sched_barrier(0);  // one pair of blocks at a time (registers)
+      };
+#pragma unroll
+      for (int rb = 0; rb + 1 < NB; rb += 2) blocks(rb, std::integral_constant<int, 2>{});
+      if constexpr (NB % 2 == 1) blocks(NB - 1, std::integral_constant<int, 1>{});
     };
     if (tok0 + kStatTokens <= V) {
       epilogue(std::true_type{});

@@ -310,3 +310,27 @@ def test_lm_head_leaf_half_tiles_agree_bit_for_bit(device, oracle, vocab):
         # and the 64-row call is the fp32 product within bf16 rounding, with
         # the oracle's statistics of its logits
         _check_head(part, hidden, weight, rows[:60], oracle)
+
+
+@pytest.mark.parametrize("vocab", [2300, 1000])
+def test_lm_head_row_tile_sizes_agree_bit_for_bit(device, oracle, vocab):
+    """Calls above 128 rows run as row tiles of two to five 64-row units, and
+    statistics blocks go in pairs with a lone one at an odd count.  Every tile
+    size and mixture at the edges of its range gives a row the same logits and
+    statistics, bit for bit, as a 64-row call; nine vocabulary tiles (one past
+    the XCDs' even share) and four."""
+    g = torch.Generator(device=device).manual_seed(vocab)
+    hidden = torch.randn(1200, 192, device=device, generator=g).to(torch.bfloat16)
+    weight = (torch.randn(vocab, 192, device=device, generator=g) * 0.1).to(torch.bfloat16)
+    rows = torch.randperm(1200, device=device, generator=g)[:1100].to(torch.int32)
+    parts = [ops.lm_head(hidden, weight, rows[k:k + 64].contiguous()) for k in range(0, 1100, 64)]
+    want = {name: torch.cat([getattr(p, name) for p in parts])
+            for name in ("logits", "tile_stats", "row_max", "row_sum")}
+    for w in (weight, ops.pack_lm_head(weight)):
+        for n in (129, 192, 193, 257, 320, 321, 385, 640, 641, 704, 1100):
+            got = ops.lm_head(hidden, w, rows[:n].contiguous())
+            torch.cuda.synchronize()
+            assert got.status.item() == 0
+            for name, value in want.items():
+                assert torch.equal(getattr(got, name), value[:n]), (n, name)
+    _check_head(got, hidden, weight, rows, oracle)
