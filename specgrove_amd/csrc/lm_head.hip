@@ -612,6 +612,9 @@ template <bool kPacked, int NB>
 __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* smem, int vt,
                                         int r0) {
   using T = PpTile<NB>;
+  // Opaque to the optimizer, which would otherwise hoist the address
+  // arithmetic of every tile size above the choice between them and spill it.
+  asm volatile("" : "+s"(vt), "+s"(r0));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -673,11 +676,20 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
   const int a_base = wv * 8 * 1024;                // this wave's 128 token rows
   const int b_base = kWBytes + wr * NB * 1024;     // this wave's hidden rows
 
-  // The main loop and the epilogue, once per group (G known at compile time,
-  // so each copy is straight-line code: no branch chooses between product
-  // sites, which would make the compiler copy the accumulators).  A barrier
-  // counts arrivals, not instructions: both copies pass 2 steps + 2 barriers.
-  // Group A: phase 2t reads stage t and issues stage t+3, phase 2t+1
+      // acc[tb][rb][i]: token 16 tb + 4 g + i of this wave's 128, row
+      // 16 rb + n of its 16 NB (lm_head_kernel's products and order).
+      floatx4 acc[8][NB];
+#pragma unroll
+      for (int tb = 0; tb < 8; ++tb)
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) acc[tb][rb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // The main loop, once per group (G known at compile time, so each copy is
+  // straight-line code: no branch chooses between product sites, which would
+  // make the compiler copy the accumulators); the epilogue is shared, since the
+  // tile sizes' copies of it would not fit the instruction cache twice.  A
+  // barrier counts arrivals, not instructions: both copies pass 2 steps + 2
+  // barriers.  Group A: phase 2t reads stage t and issues stage t+3, phase 2t+1
   // multiplies.  Group B: one idle phase, then phase 2t+1 reads stage t and
   // issues stage t+3, phase 2t+2 multiplies.  Before the barrier that ends
   // phase p every wave waits for its own copies of the stage read in phase
@@ -694,13 +706,6 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
 #pragma unroll
       for (int i = 0; i < T::template kXCopies<G>; ++i) dma16(xk, x_off[i], stage + x_lds[i]);
     };
-    // acc[tb][rb][i]: token 16 tb + 4 g + i of this wave's 128, row
-    // 16 rb + n of its 16 NB (lm_head_kernel's products and order).
-    floatx4 acc[8][NB];
-#pragma unroll
-    for (int tb = 0; tb < 8; ++tb)
-#pragma unroll
-      for (int rb = 0; rb < NB; ++rb) acc[tb][rb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     bf16x8 fa[8], fb[NB];
     auto read_frags = [&](int t) {
       const unsigned char* st = smem + (t % kLmStages) * T::kStage;
@@ -760,78 +765,90 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
     stage_step(steps - 2, std::integral_constant<int, 0>{});
     stage_step(steps - 1, std::integral_constant<int, -1>{});
     if constexpr (G == 0) __syncthreads();  // phase 2 steps: B's last products
-    // The ring is free (every barrier above waited for the LDS reads): it
-    // becomes the output staging area.
-
-    // Epilogue (lm_head_kernel's), two 16-row blocks at a time: statistics and
-    // staging, then the blocks' rows written as whole 256-byte segments (four
-    // rows an instruction).
-    const int tok0 = v0 + 128 * wv;
-    const bool tile_live = tok0 < V;
-    const int n_tiles = (V + kStatTokens - 1) / kStatTokens;
-    unsigned char* stage = smem + wave * 2 * 16 * kOutPitch;
-    uint16_t* out = static_cast<uint16_t*>(a.logits_dev);
-    auto epilogue = [&](auto full) {
-      constexpr bool kFull = decltype(full)::value;
-      auto blocks = [&](int rb, auto count) {
-        constexpr int B = decltype(count)::value;
-        const int row0 = r0 + T::kWaveRows * wr + 16 * rb;  // the blocks' first projected row
-        const float2 mz = block_epilogue<kFull, B>(
-            acc, rb, tok0, V, g, stage + (lane & 15) * kOutPitch, 16 * kOutPitch);
-        const int row = row0 + (lane & 15) + 8 * g;  // lanes g = 0: block rb, g = 2: rb + 1
-        if ((g == 0 || (B == 2 && g == 2)) && tile_live && row < a.num_rows) {
-          float* dst =
-              a.tile_stats_dev + (static_cast<int64_t>(row) * n_tiles + tok0 / kStatTokens) * 2;
-          *reinterpret_cast<float2*>(dst) = mz;
-        }
-        __builtin_amdgcn_wave_barrier();
-        const int chunk = lane & 15;
-        const int tok = tok0 + 8 * chunk;
-#pragma unroll
-        for (int i = 0; i < 4 * B; ++i) {
-          const int out_row = row0 + 4 * i + (lane >> 4);
-          const uint4 v = *reinterpret_cast<const uint4*>(
-              stage + (4 * i + (lane >> 4)) * kOutPitch + 16 * chunk);
-          if (out_row >= a.num_rows || (!kFull && tok >= V)) continue;
-          uint16_t* dst = out + static_cast<int64_t>(out_row) * a.logits_row_stride + tok;
-          if (kFull || tok + 8 <= V) {
-            *reinterpret_cast<uint4*>(dst) = v;
-          } else {
-            for (int e = 0; tok + e < V; ++e) {
-              const uint32_t w =
-                  (e >> 1) == 0 ? v.x : (e >> 1) == 1 ? v.y : (e >> 1) == 2 ? v.z : v.w;
-              dst[e] = static_cast<uint16_t>((e & 1) ? (w >> 16) : (w & 0xffffu));
-            }
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one pair of blocks at a time (registers)
-      };
-#pragma unroll
-      for (int rb = 0; rb + 1 < NB; rb += 2) blocks(rb, std::integral_constant<int, 2>{});
-      if constexpr (NB % 2 == 1) blocks(NB - 1, std::integral_constant<int, 1>{});
-    };
-    if (tok0 + kStatTokens <= V) {
-      epilogue(std::true_type{});
-    } else {
-      epilogue(std::false_type{});
-    }
   };
   if (grp == 0) {
     body(std::integral_constant<int, 0>{});
   } else {
     body(std::integral_constant<int, 1>{});
   }
+  // The ring is free (every barrier above waited for the LDS reads): it
+  // becomes the output staging area.
+
+  // Epilogue (lm_head_kernel's), two 16-row blocks at a time: statistics and
+  // staging, then the blocks' rows written as whole 256-byte segments (four
+  // rows an instruction).
+  const int tok0 = v0 + 128 * wv;
+  const bool tile_live = tok0 < V;
+  const int n_tiles = (V + kStatTokens - 1) / kStatTokens;
+  unsigned char* stage = smem + wave * 2 * 16 * kOutPitch;
+  uint16_t* out = static_cast<uint16_t*>(a.logits_dev);
+  auto epilogue = [&](auto full) {
+    constexpr bool kFull = decltype(full)::value;
+    auto blocks = [&](int rb, auto count) {
+      constexpr int B = decltype(count)::value;
+      const int row0 = r0 + T::kWaveRows * wr + 16 * rb;  // the blocks' first projected row
+      const float2 mz = block_epilogue<kFull, B>(
+          acc, rb, tok0, V, g, stage + (lane & 15) * kOutPitch, 16 * kOutPitch);
+      const int row = row0 + (lane & 15) + 8 * g;  // lanes g = 0: block rb, g = 2: rb + 1
+      if ((g == 0 || (B == 2 && g == 2)) && tile_live && row < a.num_rows) {
+        float* dst =
+            a.tile_stats_dev + (static_cast<int64_t>(row) * n_tiles + tok0 / kStatTokens) * 2;
+        *reinterpret_cast<float2*>(dst) = mz;
+      }
+      __builtin_amdgcn_wave_barrier();
+      const int chunk = lane & 15;
+      const int tok = tok0 + 8 * chunk;
+#pragma unroll
+      for (int i = 0; i < 4 * B; ++i) {
+        const int out_row = row0 + 4 * i + (lane >> 4);
+        const uint4 v = *reinterpret_cast<const uint4*>(
+            stage + (4 * i + (lane >> 4)) * kOutPitch + 16 * chunk);
+        if (out_row >= a.num_rows || (!kFull && tok >= V)) continue;
+        uint16_t* dst = out + static_cast<int64_t>(out_row) * a.logits_row_stride + tok;
+        if (kFull || tok + 8 <= V) {
+          *reinterpret_cast<uint4*>(dst) = v;
+        } else {
+          for (int e = 0; tok + e < V; ++e) {
+            const uint32_t w =
+                (e >> 1) == 0 ? v.x : (e >> 1) == 1 ? v.y : (e >> 1) == 2 ? v.z : v.w;
+            dst[e] = static_cast<uint16_t>((e & 1) ? (w >> 16) : (w & 0xffffu));
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one pair of blocks at a time (registers)
+    };
+#pragma unroll
+    for (int rb = 0; rb + 1 < NB; rb += 2) blocks(rb, std::integral_constant<int, 2>{});
+    if constexpr (NB % 2 == 1) blocks(NB - 1, std::integral_constant<int, 1>{});
+  };
+  if (tok0 + kStatTokens <= V) {
+    epilogue(std::true_type{});
+  } else {
+    epilogue(std::false_type{});
+  }
 }
 
 // Workgroup b -> (vocabulary tile, row tile).  The row tiles of one vocabulary
 // tile take consecutive slots of one XCD (tile_of); the last vocabulary tiles,
 // fewer than one per XCD, go round the XCDs one row tile at a time, so that no
-// XCD has more than one workgroup more than another.
+// XCD has more than one workgroup more than another.  The tiles from `whole`
+// on, a last round that would leave more than half of the CUs idle, run as two
+// row halves each, eight workgroups apart (the same XCD): one such round of 594
+// tiles (V 151,936, H 4096) took 256 rows from 385 to 355 us, 300 rows from 431
+// to 392; 473 rows at V 43,748, H 512 from 58 to 46.5.
 template <bool kPacked>
 __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs a, int v_tiles,
-                                                                    int r_tiles, int units) {
+                                                                    int r_tiles, int units,
+                                                                    int whole) {
   __shared__ __align__(1024) unsigned char smem[kPpLds];
-  const int b = static_cast<int>(blockIdx.x);
+  int b = static_cast<int>(blockIdx.x);
+  int half = -1;
+  if (b >= whole) {
+    const int k = b - whole;
+    half = (k / kLmXcds) & 1;
+    b = whole + k / (2 * kLmXcds) * kLmXcds + k % kLmXcds;
+    if (b >= v_tiles * r_tiles) return;
+  }
   const int v_even = v_tiles / kLmXcds * kLmXcds;
   int vt, rt;
   if (b < v_even * r_tiles) {
@@ -843,11 +860,18 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
   }
   int r0, nb;
   row_tile(units, r_tiles, rt, r0, nb);
+  if (half == 0) {
+    nb = (nb + 1) / 2;
+  } else if (half == 1) {
+    r0 += 64 * ((nb + 1) / 2);
+    nb = nb / 2;
+  }
   switch (nb) {
     case 5: pp_tile<kPacked, 5>(a, smem, vt, r0); break;
     case 4: pp_tile<kPacked, 4>(a, smem, vt, r0); break;
     case 3: pp_tile<kPacked, 3>(a, smem, vt, r0); break;
-    default: pp_tile<kPacked, 2>(a, smem, vt, r0); break;
+    case 2: pp_tile<kPacked, 2>(a, smem, vt, r0); break;
+    default: pp_tile<kPacked, 1>(a, smem, vt, r0); break;
   }
 }
 
@@ -964,14 +988,24 @@ int launch_lm_head(const SgLmHeadArgs& a, bool packed, hipStream_t s) {
   auto launch_pp = [&]() -> int {
     const int units = (a.num_rows + 63) / 64;  // >= 3: every tile has two units or more
     const int r_tiles = (units + kPpMaxUnits - 1) / kPpMaxUnits;
-    const int64_t blocks = static_cast<int64_t>(v_tiles) * r_tiles;
+    const int64_t tiles = static_cast<int64_t>(v_tiles) * r_tiles;
+    SG_REQUIRE(tiles < INT32_MAX, "wave too large");
+    int64_t blocks = tiles;
+    int64_t whole = tiles;
+    // A half round or less of tiles left over: as row halves (one workgroup of
+    // this kernel fills a CU, so a round is one per CU).
+    const int64_t last = tiles % kRoundCUs;
+    if (last > 0 && last <= kRoundCUs / 2) {
+      whole = tiles - last;
+      blocks = whole + (last + kLmXcds - 1) / kLmXcds * kLmXcds * 2;
+    }
     SG_REQUIRE(blocks < INT32_MAX, "wave too large");
     if (packed) {
       lm_head_pp_kernel<true><<<dim3(static_cast<unsigned>(blocks)), dim3(kPpThreads), 0, s>>>(
-          a, v_tiles, r_tiles, units);
+          a, v_tiles, r_tiles, units, static_cast<int>(whole));
     } else {
       lm_head_pp_kernel<false><<<dim3(static_cast<unsigned>(blocks)), dim3(kPpThreads), 0, s>>>(
-          a, v_tiles, r_tiles, units);
+          a, v_tiles, r_tiles, units, static_cast<int>(whole));
     }
     SG_LAUNCH_CHECK();
     return SG_OK;

@@ -312,13 +312,14 @@ def test_lm_head_leaf_half_tiles_agree_bit_for_bit(device, oracle, vocab):
         _check_head(part, hidden, weight, rows[:60], oracle)
 
 
-@pytest.mark.parametrize("vocab", [2300, 1000])
+@pytest.mark.parametrize("vocab", [2300, 1000, 33000])
 def test_lm_head_row_tile_sizes_agree_bit_for_bit(device, oracle, vocab):
     """Calls above 128 rows run as row tiles of two to five 64-row units, and
     statistics blocks go in pairs with a lone one at an odd count.  Every tile
     size and mixture at the edges of its range gives a row the same logits and
-    statistics, bit for bit, as a 64-row call; nine vocabulary tiles (one past
-    the XCDs' even share) and four."""
+    statistics, bit for bit, as a 64-row call.  Nine vocabulary tiles (one past
+    the XCDs' even share) and four: every tile runs as two row halves of one
+    to three units; 129: whole tiles, and both in calls of two row tiles."""
     g = torch.Generator(device=device).manual_seed(vocab)
     hidden = torch.randn(1200, 192, device=device, generator=g).to(torch.bfloat16)
     weight = (torch.randn(vocab, 192, device=device, generator=g) * 0.1).to(torch.bfloat16)
