@@ -366,6 +366,12 @@ int sg_lm_head_pack_weight(const void* weight_dev, int64_t weight_row_stride, in
  * 1 KiB), larger calls about 5 % faster. */
 int sg_lm_head_packed(const SgLmHeadArgs* args, sg_stream_t stream);
 
+/* sg_lm_head (packed 0) or sg_lm_head_packed (otherwise), except that the call
+ * writes *status_dev: 0, or SG_EINVAL when a row index lies outside
+ * [0, num_hidden_rows) (nothing is written when num_rows is 0).  For callers
+ * whose status word is new in each call: no launch clears it first. */
+int sg_lm_head_fresh(const SgLmHeadArgs* args, int32_t packed, sg_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * (E) Target decoder layer stack: the fused elementwise stages between the
  * library projections (Qwen3 family).

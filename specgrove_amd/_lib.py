@@ -138,7 +138,7 @@ EXPORTED_SYMBOLS = (
     "sg_clock_probe", "sg_wall_clock_khz",
     "sg_tree_sample_noalloc", "sg_tree_attn_plan_check", "sg_kv_split",
     "sg_lm_head", "sg_lm_head_tile_count", "sg_lm_head_packed", "sg_lm_head_pack_weight",
-    "sg_lm_head_packed_bytes",
+    "sg_lm_head_packed_bytes", "sg_lm_head_fresh",
     "sg_add_rmsnorm", "sg_qk_norm_rope", "sg_silu_mul", "sg_gather_rows",
 )
 
@@ -197,6 +197,8 @@ def load() -> ctypes.CDLL:
     lib.sg_lm_head_tile_count.argtypes = [c_i32]
     lib.sg_lm_head_packed.restype = c_i32
     lib.sg_lm_head_packed.argtypes = [ctypes.POINTER(SgLmHeadArgs), c_void_p]
+    lib.sg_lm_head_fresh.restype = c_i32
+    lib.sg_lm_head_fresh.argtypes = [ctypes.POINTER(SgLmHeadArgs), c_i32, c_void_p]
     lib.sg_lm_head_pack_weight.restype = c_i32
     lib.sg_lm_head_pack_weight.argtypes = [c_void_p, c_i64, c_i32, c_i32, c_void_p, c_void_p]
     lib.sg_lm_head_packed_bytes.restype = c_i64

@@ -55,6 +55,7 @@
 #include <algorithm>
 #include <climits>
 #include <type_traits>
+#include <utility>
 
 #include "sg_common.h"
 #include "sg_math.h"
@@ -877,7 +878,20 @@ __global__ __launch_bounds__(kPpThreads, 1) void lm_head_pp_kernel(SgLmHeadArgs 
 
 // Row (max, sum) from the tile pairs: one wave per row; lane l merges tiles
 // l, l+64, ... in increasing order, then the xor butterfly merges the lanes.
-__global__ __launch_bounds__(kMergeRowsPerBlock * kWave) void lm_head_rows_kernel(SgLmHeadArgs a) {
+// With status_out the first workgroup also checks every row index and writes
+// the call's status.
+__global__ __launch_bounds__(kMergeRowsPerBlock * kWave) void lm_head_rows_kernel(
+    SgLmHeadArgs a, int32_t* status_out) {
+  if (blockIdx.x == 0 && status_out != nullptr) {
+    bool bad = false;
+    for (int r = threadIdx.x; a.row_index_dev != nullptr && r < a.num_rows;
+         r += kMergeRowsPerBlock * kWave) {
+      const int src = a.row_index_dev[r];
+      bad = bad || src < 0 || src >= a.num_hidden_rows;
+    }
+    const int any = __syncthreads_or(bad);
+    if (threadIdx.x == 0) *status_out = any ? SG_EINVAL : SG_OK;
+  }
   const int row = blockIdx.x * kMergeRowsPerBlock + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= a.num_rows) return;
@@ -960,7 +974,8 @@ int check_lm_head(const SgLmHeadArgs& a, bool packed) {
   return SG_OK;
 }
 
-int launch_lm_head(const SgLmHeadArgs& a, bool packed, hipStream_t s) {
+// status_out: written by the call (a.status_dev is only ever raised).
+int launch_lm_head(const SgLmHeadArgs& a, bool packed, int32_t* status_out, hipStream_t s) {
   const int v_tiles = (a.vocab + kTileV - 1) / kTileV;
   auto launch = [&](auto tag) -> int {
     constexpr int R = decltype(tag)::value;
@@ -1018,7 +1033,8 @@ int launch_lm_head(const SgLmHeadArgs& a, bool packed, hipStream_t s) {
                                      : launch(std::integral_constant<int, 4>{});
   if (rc != SG_OK) return rc;
   const int merge_blocks = (a.num_rows + kMergeRowsPerBlock - 1) / kMergeRowsPerBlock;
-  lm_head_rows_kernel<<<dim3(merge_blocks), dim3(kMergeRowsPerBlock * kWave), 0, s>>>(a);
+  lm_head_rows_kernel<<<dim3(merge_blocks), dim3(kMergeRowsPerBlock * kWave), 0, s>>>(
+      a, status_out);
   SG_LAUNCH_CHECK();
   return SG_OK;
 }
@@ -1030,19 +1046,31 @@ extern "C" int64_t sg_lm_head_tile_count(int32_t vocab) {
   return vocab >= 1 ? (static_cast<int64_t>(vocab) + sg::kStatTokens - 1) / sg::kStatTokens : -1;
 }
 
-extern "C" int sg_lm_head(const SgLmHeadArgs* args, sg_stream_t stream) {
-  using namespace sg;
+namespace sg {
+namespace {
+
+// One call: `fresh` writes *status_dev, otherwise it is only raised.
+int run_lm_head(const SgLmHeadArgs* args, bool packed, bool fresh, sg_stream_t stream) {
   clear_error();
   SG_REQUIRE(args != nullptr, "null args");
-  const SgLmHeadArgs& a = *args;
+  SgLmHeadArgs a = *args;
   SG_REQUIRE(a.num_rows >= 0, "num_rows must be non-negative");
   SG_REQUIRE(a.vocab >= 1, "vocab must be positive");
   SG_REQUIRE(a.hidden_size >= 2 * kStepK && a.hidden_size % (2 * kStepK) == 0,
              "hidden_size must be a positive multiple of 64");
   if (a.num_rows == 0) return SG_OK;
-  const int rc = check_lm_head(a, false);
+  const int rc = check_lm_head(a, packed);
   if (rc != SG_OK) return rc;
-  return launch_lm_head(a, false, static_cast<hipStream_t>(stream));
+  int32_t* status_out = nullptr;
+  if (fresh) std::swap(status_out, a.status_dev);
+  return launch_lm_head(a, packed, status_out, static_cast<hipStream_t>(stream));
+}
+
+}  // namespace
+}  // namespace sg
+
+extern "C" int sg_lm_head(const SgLmHeadArgs* args, sg_stream_t stream) {
+  return sg::run_lm_head(args, false, false, stream);
 }
 
 extern "C" int64_t sg_lm_head_packed_bytes(int32_t vocab, int32_t hidden_size) {
@@ -1077,16 +1105,9 @@ extern "C" int sg_lm_head_pack_weight(const void* weight_dev, int64_t weight_row
 }
 
 extern "C" int sg_lm_head_packed(const SgLmHeadArgs* args, sg_stream_t stream) {
-  using namespace sg;
-  clear_error();
-  SG_REQUIRE(args != nullptr, "null args");
-  const SgLmHeadArgs& a = *args;
-  SG_REQUIRE(a.num_rows >= 0, "num_rows must be non-negative");
-  SG_REQUIRE(a.vocab >= 1, "vocab must be positive");
-  SG_REQUIRE(a.hidden_size >= 2 * kStepK && a.hidden_size % (2 * kStepK) == 0,
-             "hidden_size must be a positive multiple of 64");
-  if (a.num_rows == 0) return SG_OK;
-  const int rc = check_lm_head(a, true);
-  if (rc != SG_OK) return rc;
-  return launch_lm_head(a, true, static_cast<hipStream_t>(stream));
+  return sg::run_lm_head(args, true, false, stream);
+}
+
+extern "C" int sg_lm_head_fresh(const SgLmHeadArgs* args, int32_t packed, sg_stream_t stream) {
+  return sg::run_lm_head(args, packed != 0, true, stream);
 }

@@ -546,6 +546,15 @@ __device__ void route_request(const SgTreeSampleArgs& a, int req, int r0, int n,
   __syncthreads();
 }
 
+// Request req's record in the workspace.
+__device__ __forceinline__ int32_t* request_record(const SgTreeSampleArgs& a, int req) {
+  const int slabs = (a.vocab + kSlab - 1) / kSlab;
+  return reinterpret_cast<int32_t*>(static_cast<float*>(a.workspace_dev) +
+                                    static_cast<int64_t>(a.num_requests) * slabs *
+                                        (1 + kLinesPerSlab)) +
+         static_cast<int64_t>(req) * kRecordInts;
+}
+
 // Walk, part 1.  Grid (request, chunk of kWalkWaves slabs); every workgroup
 // routes its request (cheap, LDS only), workgroup chunk 0 writes the accepted
 // nodes, accept length and keep rows, and every wave computes the complement
@@ -571,7 +580,7 @@ __global__ __launch_bounds__(kWalkThreads) void exit_totals_kernel(SgTreeSampleA
       a.accept_len_dev[req] = -1;
       a.bonus_dev[req] = -1;
       if (a.terminal_leaf_dev) a.terminal_leaf_dev[req] = -1;
-      if (a.status_dev) atomicExch(a.status_dev, SG_EINVAL);
+      request_record(a, req)[0] = -1;
     }
     return;
   }
@@ -588,10 +597,7 @@ __global__ __launch_bounds__(kWalkThreads) void exit_totals_kernel(SgTreeSampleA
       a.accept_len_dev[req] = sh.broken ? -1 : sh.depth;
       if (a.terminal_leaf_dev)
         a.terminal_leaf_dev[req] = (!sh.broken && exit_row < 0) ? sh.exit_node : -1;
-      if (sh.broken) {
-        a.bonus_dev[req] = -1;
-        if (a.status_dev) atomicExch(a.status_dev, SG_EINVAL);
-      }
+      if (sh.broken) a.bonus_dev[req] = -1;
     }
     if (a.keep_rows_dev) {
       __syncthreads();  // nodes_out written by thread 0
@@ -599,11 +605,7 @@ __global__ __launch_bounds__(kWalkThreads) void exit_totals_kernel(SgTreeSampleA
       for (int k = tid; k <= a.max_depth; k += blockDim.x)
         keep[k] = (k == 0) ? 0 : (!sh.broken && k <= sh.depth ? nodes_out[k - 1] : -1);
     }
-    const int slabs_all = (a.vocab + kSlab - 1) / kSlab;
-    int32_t* rec = reinterpret_cast<int32_t*>(static_cast<float*>(a.workspace_dev) +
-                                              static_cast<int64_t>(a.num_requests) * slabs_all *
-                                                  (1 + kLinesPerSlab)) +
-                   static_cast<int64_t>(req) * kRecordInts;
+    int32_t* rec = request_record(a, req);
     if (tid == 0) {
       rec[0] = sh.broken ? -1 : sh.depth;
       rec[1] = sh.exit_node;
@@ -656,10 +658,7 @@ __global__ __launch_bounds__(kWave) void exit_find_kernel(SgTreeSampleArgs a) {
   const float* __restrict__ line_totals = static_cast<const float*>(a.workspace_dev) +
                                           static_cast<int64_t>(a.num_requests) * slabs +
                                           static_cast<int64_t>(req) * slabs * kLinesPerSlab;
-  const int32_t* rec = reinterpret_cast<const int32_t*>(
-                           static_cast<const float*>(a.workspace_dev) +
-                           static_cast<int64_t>(a.num_requests) * slabs * (1 + kLinesPerSlab)) +
-                       static_cast<int64_t>(req) * kRecordInts;
+  const int32_t* rec = request_record(a, req);
   const float* __restrict__ u = a.uniforms_dev + static_cast<int64_t>(a.uniform_stride) * req;
   // One round trip: the row range, part 1's record (accept length, child
   // count, exit row), the first 64 child tokens and the slab totals.
@@ -672,9 +671,19 @@ __global__ __launch_bounds__(kWave) void exit_find_kernel(SgTreeSampleArgs a) {
 #pragma unroll
   for (int q = 0; q < (kMaxSlabs + kWave - 1) / kWave; ++q)
     tot[q] = q * kWave + lane < slabs ? totals[q * kWave + lane] : 0.0f;
-  // The record exists only for a valid tree; part 1 reported the others.
+  // Every request's record says whether its walk broke the contract: one wave
+  // gives the call's status word its value (a launch to clear it before part 1
+  // raised it cost 5 us a call).
+  if (req == 0 && a.status_dev != nullptr) {
+    bool broken = false;
+    for (int i = lane; i < a.num_requests; i += kWave)
+      broken = broken || request_record(a, i)[0] < 0;
+    const bool any = __ballot(broken) != 0;
+    if (lane == 0) *a.status_dev = any ? SG_EINVAL : SG_OK;
+  }
+  // The record is whole only for a valid tree.
   if (n < 1 || n > kMaxTreeRows || r0 < 0 || r0 > a.num_rows - n) return;
-  if (depth < 0) return;  // broken walk, reported by part 1
+  if (depth < 0) return;  // broken walk
   const int exit_row = rec[3];
   if (exit_row < 0) {      // terminal leaf without a projected row
     if (lane == 0) a.bonus_dev[req] = -1;
@@ -1109,7 +1118,7 @@ int check_sample_args(const SgTreeSampleArgs* args) {
   return SG_OK;
 }
 
-// Enqueues the three kernels of one sampling call; a.workspace_dev holds at
+// Enqueues the two kernels of one sampling call; a.workspace_dev holds at
 // least sg_tree_sample_workspace_bytes(num_requests, statistics rows, vocab) bytes.
 int64_t stats_rows_of(const SgTreeSampleArgs& a) {
   return (a.flags & SG_SAMPLE_STATS_READY) ? 0
@@ -1117,17 +1126,19 @@ int64_t stats_rows_of(const SgTreeSampleArgs& a) {
 }
 
 int launch_tree_sample(const SgTreeSampleArgs& a, hipStream_t s) {
-  // With SG_SAMPLE_STATS_READY the statistics pass only clears the status and
-  // the complement draw runs (exit_totals + exit_find); otherwise the pass
-  // keeps every row's slab pairs and one kernel walks and draws.
+  // With SG_SAMPLE_STATS_READY the complement draw runs (exit_totals +
+  // exit_find, which writes the status); otherwise the statistics pass clears
+  // the status and keeps every row's slab pairs, and one kernel walks and draws.
   const bool ready = (a.flags & SG_SAMPLE_STATS_READY) != 0;
   const int stats_rows = static_cast<int>(stats_rows_of(a));
   float* slab_stats = static_cast<float*>(a.workspace_dev) +
                       request_region_floats(a.num_requests, a.vocab);
-  int rc = launch_row_stats(a.logits_dev, a.logits_dtype, a.logits_row_stride, a.vocab,
-                            stats_rows, a.row_max_dev, a.row_sum_dev,
-                            ready ? nullptr : slab_stats, a.status_dev, s);
-  if (rc != SG_OK) return rc;
+  if (!ready) {
+    const int rc = launch_row_stats(a.logits_dev, a.logits_dtype, a.logits_row_stride, a.vocab,
+                                    stats_rows, a.row_max_dev, a.row_sum_dev, slab_stats,
+                                    a.status_dev, s);
+    if (rc != SG_OK) return rc;
+  }
   const int slabs = (a.vocab + kSlab - 1) / kSlab;
   const dim3 grid1(a.num_requests, (slabs + kWalkWaves - 1) / kWalkWaves);
   hipError_t err = hipSuccess;

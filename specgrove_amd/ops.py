@@ -428,6 +428,13 @@ _LOGITS_DTYPES = {torch.float32: _lib.SG_DTYPE_F32, torch.bfloat16: _lib.SG_DTYP
                   torch.float16: _lib.SG_DTYPE_F16}
 
 
+def _new_status(work: int, device) -> torch.Tensor:
+    """A call's status word.  The call writes it when it has work (requests or
+    rows), so no fill kernel runs first."""
+    make = torch.empty if work > 0 else torch.zeros
+    return make(1, dtype=torch.int32, device=device)
+
+
 def _check_logits(logits: torch.Tensor) -> int:
     _require(isinstance(logits, torch.Tensor) and logits.is_cuda,
              "logits must be a HIP device tensor")
@@ -522,7 +529,7 @@ def tree_sample(logits: torch.Tensor, row_offset: torch.Tensor, parent: torch.Te
             keep_rows=torch.empty((n, max_depth + 1), dtype=torch.int32, device=dev),
             row_max=torch.empty(rows, dtype=torch.float32, device=dev),
             row_sum=torch.empty(rows, dtype=torch.float32, device=dev),
-            status=torch.zeros(1, dtype=torch.int32, device=dev),
+            status=_new_status(n, dev),
         )
     else:
         _check_sample_out(out, n, rows, max_depth)
@@ -605,7 +612,7 @@ def tree_sample_projected(logits: torch.Tensor, row_offset: torch.Tensor, parent
         bonus=torch.empty(n, dtype=torch.int32, device=dev),
         keep_rows=torch.empty((n, max_depth + 1), dtype=torch.int32, device=dev),
         terminal_leaf=torch.empty(n, dtype=torch.int32, device=dev),
-        status=torch.zeros(1, dtype=torch.int32, device=dev),
+        status=_new_status(n, dev),
         workspace=torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev))
     a = _sample_args(logits, row_offset, parent, token, uniforms, max_depth, out, n, rows,
                      out.workspace)
@@ -767,7 +774,7 @@ def lm_head(hidden: torch.Tensor, weight,
         tile_stats=torch.empty((rows, tiles, 2), dtype=torch.float32, device=dev),
         row_max=torch.empty(rows, dtype=torch.float32, device=dev),
         row_sum=torch.empty(rows, dtype=torch.float32, device=dev),
-        status=torch.zeros(1, dtype=torch.int32, device=dev))
+        status=_new_status(rows, dev))
     a = _lib.SgLmHeadArgs()
     a.num_rows = rows
     a.hidden_size = hsize
@@ -784,6 +791,6 @@ def lm_head(hidden: torch.Tensor, weight,
     a.row_max_dev = res.row_max.data_ptr()
     a.row_sum_dev = res.row_sum.data_ptr()
     a.status_dev = res.status.data_ptr()
-    name = "sg_lm_head_packed" if packed else "sg_lm_head"
-    _lib.check(getattr(_lib.load(), name)(ctypes.byref(a), _stream_handle()), name)
+    _lib.check(_lib.load().sg_lm_head_fresh(ctypes.byref(a), int(packed), _stream_handle()),
+               "sg_lm_head_packed" if packed else "sg_lm_head")
     return res

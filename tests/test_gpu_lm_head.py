@@ -335,3 +335,43 @@ def test_lm_head_row_tile_sizes_agree_bit_for_bit(device, oracle, vocab):
             for name, value in want.items():
                 assert torch.equal(getattr(got, name), value[:n]), (n, name)
     _check_head(got, hidden, weight, rows, oracle)
+
+
+@pytest.mark.parametrize("rows,bad", [(1, 0), (70, 69), (300, 299), (300, None)])
+def test_lm_head_writes_its_status(device, rows, bad):
+    """The call gives its status word its value, whatever the word held: the
+    first workgroup of the row merge checks every index (256 threads, then a
+    second round)."""
+    hidden, weight = _inputs(device, 64, 64, 300, seed=rows)
+    index = torch.randint(0, 64, (rows,), device=device, dtype=torch.int32)
+    if bad is not None:
+        index[bad] = 64
+    junk = torch.full((1 << 12,), 7, dtype=torch.int32, device=device)
+    del junk  # the allocator hands its bytes to the next words
+    assert int(ops.lm_head(hidden, weight, index).status.item()) == (0 if bad is None else -1)
+
+
+@pytest.mark.parametrize("requests", [3, 65, 130])
+def test_projected_walk_writes_its_status(device, requests):
+    """One broken request anywhere (also past the 64 that one round of the
+    status check reads) makes the call's status SG_EINVAL; none, SG_OK."""
+    vocab, g = 300, torch.Generator(device=device).manual_seed(requests)
+    logits = torch.randn(2 * requests, vocab, device=device, generator=g).to(torch.bfloat16)
+    m, z = ops.row_stats(logits)
+    offset = torch.arange(requests + 1, device=device, dtype=torch.int32) * 2
+    parent = torch.tensor([-1, 0] * requests, device=device, dtype=torch.int32)
+    uniforms = torch.rand(requests, 4, device=device, generator=g)
+    for broken in (None, requests - 1, 0, None):
+        token = torch.ones(2 * requests, dtype=torch.int32, device=device)
+        if broken is not None:
+            token[2 * broken + 1] = vocab  # outside the vocabulary
+        r = ops.tree_sample_projected(logits, offset, parent, token, uniforms, 1, row_max=m,
+                                      row_sum=z)
+        assert int(r.status.item()) == (0 if broken is None else -1), broken
+        want = (r.accept_len == -1).nonzero().flatten().tolist()
+        assert want == ([] if broken is None else [broken])
+    short = offset.clone()
+    short[-1] = 2 * requests + 1  # the last request's rows run past the packed rows
+    r = ops.tree_sample_projected(logits, short, parent, torch.ones_like(parent), uniforms, 1,
+                                  row_max=m, row_sum=z)
+    assert int(r.status.item()) == -1 and int(r.accept_len[-1]) == -1
