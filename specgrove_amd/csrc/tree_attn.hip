@@ -301,7 +301,7 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   __shared__ __align__(1024) unsigned char s_k[kStages * STAGEB];
   __shared__ __align__(1024) unsigned char s_v[kStages * STAGEB];
   __shared__ uint32_t s_anc[kQPerUnit][kAncWords];
-  __shared__ int s_parent[kMaxTreeRows];
+  __shared__ int2 s_run[kMaxTreeRows];  // first node of each node's run, and that node's parent
 
   const int G = a.num_q_heads / a.num_kv_heads;
   const int tid = threadIdx.x;
@@ -347,9 +347,24 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   // tile and the planner did not split the rows (flags bit 1).
   const bool stream_kv = (u.flags & 2) == 0 && n * G <= kQPerUnit;
 
-  // Ancestor-or-self bitsets of the tile's rows (request-local numbering).
+  // Ancestor-or-self bitsets of the tile's rows (request-local numbering).  A
+  // row's walk to its root takes a run of consecutive nodes (parent = node - 1)
+  // at a step: every step is a dependent LDS read and eight words of bits, and
+  // a 256-row prompt chunk walked node by node spent ~17 us here, an eighth of
+  // its unit.  Runs are found inside groups of 64 nodes (a ballot per wave), so
+  // a chain of 256 takes four steps and a bushy tree never more than its depth.
+  // With the tree tiles that a row tile cannot see left out (below), eight
+  // 256-row chunks at 483-3,006 cached tokens (32 q / 8 kv heads): 138 -> 110 us.
   if (do_tree) {
-    for (int k = tid; k < n; k += kThreads) s_parent[k] = a.parent_dev[r0 + k];
+    {
+      // One node per thread (n <= kMaxTreeRows = kThreads).
+      const int p = tid < n ? a.parent_dev[r0 + tid] : -1;
+      const uint64_t linked = __ballot(lane > 0 && p == tid - 1);
+      // The run starts at the highest unlinked lane at or below this one.
+      const int start = 63 - __builtin_clzll(~linked & (~0ull >> (63 - lane)));
+      const int above = __shfl(p, start);
+      s_run[tid] = make_int2((tid & ~63) + start, above);
+    }
     for (int k = tid; k < kQPerUnit * kAncWords; k += kThreads) (&s_anc[0][0])[k] = 0u;
     __syncthreads();
     if (tid < u.row_count) {
@@ -358,11 +373,14 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
 #pragma unroll
       for (int w = 0; w < kAncWords; ++w) bits[w] = 0u;
       for (int guard = 0; node >= 0 && guard < kMaxTreeRows; ++guard) {
+        const int2 run = s_run[node];
 #pragma unroll
-        for (int w = 0; w < kAncWords; ++w)
-          bits[w] |= (w == (node >> 5)) ? (1u << (node & 31)) : 0u;
-        const int p = s_parent[node];
-        node = (p < node) ? p : -1;
+        for (int w = 0; w < kAncWords; ++w) {
+          // Bits run.x .. node of word w.
+          const int lo = max(run.x - 32 * w, 0), hi = min(node - 32 * w, 31);
+          bits[w] |= lo <= hi ? (0xffffffffu << (lo & 31)) & (0xffffffffu >> ((31 - hi) & 31)) : 0u;
+        }
+        node = (run.y < run.x) ? run.y : -1;
       }
 #pragma unroll
       for (int w = 0; w < kAncWords; ++w) s_anc[tid][w] = bits[w];
@@ -382,7 +400,10 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   const int prefix_keys = u.key_end - u.key_begin;
   const int tiles_prefix = (prefix_keys + kTileKeys - 1) / kTileKeys;
   const int tiles_full = prefix_keys / kTileKeys;
-  const int tiles_tree = do_tree ? (n + kTileKeys - 1) / kTileKeys : 0;
+  // Parents precede their children, so no row of the unit sees a tree key
+  // behind the unit's last row.
+  const int tree_keys = u.row_begin + u.row_count;
+  const int tiles_tree = do_tree ? (tree_keys + kTileKeys - 1) / kTileKeys : 0;
   const int tiles = tiles_prefix + tiles_tree;
   const int64_t prefix0 = a.prefix_start_dev[u.req] + u.key_begin;
   const uint16_t* kc = static_cast<const uint16_t*>(a.k_cache_dev) + g * a.cache_head_stride +

@@ -120,6 +120,33 @@ def test_qwen3_8b_full_size_sampled_requests_and_isolation(device, oracle):
     assert not torch.equal(poisoned[~keep], got[~keep])
 
 
+def _run_tree(nodes, run, offset):
+    """Runs of consecutive nodes; each run hangs under an earlier node that is
+    mostly not its predecessor."""
+    parents = [-1]
+    for k in range(1, nodes):
+        parents.append(k - 1 if (k + offset) % run else max(0, k - 1 - (k * 7) % (k + 1)))
+    return parents
+
+
+@pytest.mark.parametrize("nodes,run,offset", [
+    (256, 1000, 0), (255, 1000, 0),              # one chain, over all 64-node groups
+    (256, 64, 0), (256, 64, 63), (200, 63, 1),   # runs that end at, before, after a group
+    (65, 1000, 0), (64, 2, 0), (33, 1, 0), (1, 1, 0)])
+def test_runs_of_consecutive_nodes_and_unseen_tree_tiles(device, oracle, nodes, run, offset):
+    # 4 q / 2 kv heads: row tiles of 64 rows, so the earlier tiles of the larger
+    # trees skip the tree keys behind their last row.
+    tree = _run_tree(nodes, run, offset)
+    lengths = np.asarray([40, 0, 130], np.int32)
+    wl = W.AttentionWorkload("runs", 4, 2, 64, lengths, [tree, tree[:max(1, nodes // 2)], tree],
+                             [[0] * (n - 1) for n in (nodes, max(1, nodes // 2), nodes)], 448)
+    tensors, dev, meta = _inputs(wl, device, nodes + run + offset)
+    got, _ = _run(wl, dev, meta, device)
+    ks, vs = _prefix_lists(wl, tensors)
+    q, kc, vc, kt, vt = tensors
+    _assert_close(got, oracle.attention_dense(q, ks, vs, kt, vt, wl.parents))
+
+
 def test_strided_query_and_output_views(device, oracle):
     wl = W.tiny_attention_workload(seed=3, num_q_heads=8, num_kv_heads=2, head_dim=128)
     tensors, dev, meta = _inputs(wl, device, 14)
