@@ -26,6 +26,15 @@
 // before the product with up.  Sums of squares run in fp32 in this kernel's
 // own order, and 1/sqrt and sincos are the device's, so a normed or rotated
 // value can still differ from transformers' by one bf16 ulp.
+//
+// All of them are bound by HBM once each load of a thread is issued before the
+// first is used and the conversions to bf16 are gfx950's own.  One layer's four
+// calls over 2,048 rows (hidden 4096, intermediate 12288, 32 q / 8 kv heads of
+// 128; 336 MB): 81.4 -> 77.4 us, and 72.8 us (4.6 TB/s, a large copy reaches 4.9)
+// with non-temporal loads.  Non-temporal stores were 3.5 us faster still here
+// and 25 us slower in a 512-row decoder of four layers, whose next kernel reads
+// the stored rows from the caches: not used.
+#include <algorithm>
 #include <cmath>
 
 #include "sg_common.h"
@@ -33,9 +42,16 @@
 namespace sg {
 namespace {
 
-constexpr int kNormThreads = 256;
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
-__device__ __forceinline__ float bf16r(float x) { return bf16_to_f32(f32_to_bf16(x)); }
+// 16 bytes that this kernel alone reads: the non-temporal hint keeps them from
+// displacing the outputs, which the next kernel reads, in the caches.
+__device__ __forceinline__ uint4 ntload(const void* p) {
+  const u32x4 v = __builtin_nontemporal_load(static_cast<const u32x4*>(p));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+constexpr int kNormThreads = 256;
 
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
 #pragma unroll
@@ -47,13 +63,24 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   float t = 0.0f;
   const int waves = blockDim.x >> 6;
   for (int w = 0; w < waves; ++w) t += scratch[w];
-  __syncthreads();
   return t;
 }
 
-// One row per workgroup; 8 bf16 (16 bytes) per thread per step.
+// The two bf16 halves of a word as floats, and both rounded to bf16 and back.
+struct Pair {
+  float lo, hi;
+};
+__device__ __forceinline__ Pair unpack(uint32_t v) {
+  return {__uint_as_float(v << 16), __uint_as_float(v & 0xffff0000u)};
+}
+__device__ __forceinline__ Pair bf16r(float lo, float hi) { return unpack(pack_bf16x2(lo, hi)); }
+
+// One row per workgroup; 8 bf16 (16 bytes) per thread and chunk, kChunks the
+// fewest chunks that hold the row, so that every load of the row (the weight's
+// too) is issued before the first is used.
 // sum = x (+ residual); residual_out = bf16(sum) when requested;
 // out = bf16(w * bf16(s * rsqrt(mean(s^2) + eps))), s = bf16(sum).
+template <int kChunks, bool kResidual>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual,
     const uint16_t* __restrict__ weight, uint16_t* __restrict__ out,
@@ -62,55 +89,62 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
   __shared__ float scratch[kNormThreads / 64];
   const int64_t row = blockIdx.x;
   const uint16_t* xr = x + row * x_stride;
-  const uint16_t* rr = residual != nullptr ? residual + row * res_stride : nullptr;
-  constexpr int kMaxChunks = 4;  // hidden <= 8192
-  uint4 s[kMaxChunks];
+  const uint16_t* rr = residual + row * res_stride;
+  uint4 s[kChunks], b[kChunks], w[kChunks];
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int e = 8 * (threadIdx.x + c * kNormThreads);
+    const bool live = e < hidden;
+    s[c] = live ? ntload(xr + e) : make_uint4(0u, 0u, 0u, 0u);
+    if (kResidual)
+      b[c] = live ? ntload(rr + e) : make_uint4(0u, 0u, 0u, 0u);
+  }
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int e = 8 * (threadIdx.x + c * kNormThreads);
+    w[c] = e < hidden ? *reinterpret_cast<const uint4*>(weight + e) : make_uint4(0u, 0u, 0u, 0u);
+  }
   float ss = 0.0f;
 #pragma unroll
-  for (int c = 0; c < kMaxChunks; ++c) {
-    const int e = 8 * (threadIdx.x + c * kNormThreads);
-    s[c] = make_uint4(0u, 0u, 0u, 0u);
-    if (e >= hidden) continue;
-    uint4 a = *reinterpret_cast<const uint4*>(xr + e);
-    if (rr != nullptr) {
-      const uint4 b = *reinterpret_cast<const uint4*>(rr + e);
-      const uint32_t av[4] = {a.x, a.y, a.z, a.w};
-      const uint32_t bv[4] = {b.x, b.y, b.z, b.w};
-      uint32_t o[4];
+  for (int c = 0; c < kChunks; ++c) {
+    uint32_t v[4] = {s[c].x, s[c].y, s[c].z, s[c].w};
+    if (kResidual) {
+      const uint32_t bv[4] = {b[c].x, b[c].y, b[c].z, b[c].w};
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float lo = bf16_to_f32(av[k] & 0xffffu) + bf16_to_f32(bv[k] & 0xffffu);
-        const float hi = bf16_to_f32(av[k] >> 16) + bf16_to_f32(bv[k] >> 16);
-        o[k] = pack_bf16x2(lo, hi);
+        const Pair p = unpack(v[k]), q = unpack(bv[k]);
+        v[k] = pack_bf16x2(p.lo + q.lo, p.hi + q.hi);
       }
-      a = make_uint4(o[0], o[1], o[2], o[3]);
+      s[c] = make_uint4(v[0], v[1], v[2], v[3]);
     }
-    s[c] = a;
-    const uint32_t v[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float lo = bf16_to_f32(v[k] & 0xffffu);
-      const float hi = bf16_to_f32(v[k] >> 16);
-      ss += lo * lo + hi * hi;
+      const Pair p = unpack(v[k]);
+      ss += p.lo * p.lo + p.hi * p.hi;
+    }
+  }
+  if (residual_out != nullptr) {
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const int e = 8 * (threadIdx.x + c * kNormThreads);
+      if (e < hidden)
+        *reinterpret_cast<uint4*>(residual_out + row * res_out_stride + e) = s[c];
     }
   }
   const float total = block_sum(ss, scratch);
   const float r = 1.0f / sqrtf(total / static_cast<float>(hidden) + eps);
 #pragma unroll
-  for (int c = 0; c < kMaxChunks; ++c) {
+  for (int c = 0; c < kChunks; ++c) {
     const int e = 8 * (threadIdx.x + c * kNormThreads);
     if (e >= hidden) continue;
-    if (residual_out != nullptr)
-      *reinterpret_cast<uint4*>(residual_out + row * res_out_stride + e) = s[c];
-    const uint4 w = *reinterpret_cast<const uint4*>(weight + e);
     const uint32_t v[4] = {s[c].x, s[c].y, s[c].z, s[c].w};
-    const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t wv[4] = {w[c].x, w[c].y, w[c].z, w[c].w};
     uint32_t o[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float lo = bf16_to_f32(wv[k] & 0xffffu) * bf16r(bf16_to_f32(v[k] & 0xffffu) * r);
-      const float hi = bf16_to_f32(wv[k] >> 16) * bf16r(bf16_to_f32(v[k] >> 16) * r);
-      o[k] = pack_bf16x2(lo, hi);
+      const Pair p = unpack(v[k]), q = unpack(wv[k]);
+      const Pair n = bf16r(p.lo * r, p.hi * r);
+      o[k] = pack_bf16x2(q.lo * n.lo, q.hi * n.hi);
     }
     *reinterpret_cast<uint4*>(out + row * out_stride + e) = make_uint4(o[0], o[1], o[2], o[3]);
   }
@@ -134,125 +168,142 @@ __global__ __launch_bounds__(kNormThreads) void qk_norm_rope_kernel(
   constexpr int H2 = D / 2;
   constexpr int LPH = D / 8;        // lanes per head
   constexpr int HPW = kWave / LPH;  // heads per wave at a time
+  constexpr int kBatch = 3;         // head groups of a wave loaded at a time
   __shared__ float s_cs[H2];
   __shared__ float s_sn[H2];
   const int64_t row = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int waves = blockDim.x >> 6;
-  const float pos = static_cast<float>(positions[row]);
-  for (int p = threadIdx.x; p < H2; p += blockDim.x) {
-    float sv, cv;
-    sincosf(pos * inv_freq[p], &sv, &cv);
-    s_cs[p] = bf16r(cv);
-    s_sn[p] = bf16r(sv);
-  }
-  __syncthreads();
   const int j = lane % LPH;             // 16-byte chunk of the head
   const int slot = lane / LPH;          // head of the wave's group
   const bool lower = j < LPH / 2;       // dims below D/2
   const int pair0 = 8 * (j % (LPH / 2));
+  const int heads = hq + 2 * hkv;
+  const uint16_t* src = qkv + row * qkv_stride + 8 * j;
+  uint4 raw[kBatch];
+  auto load = [&](int h0) {
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) {
+      const int h = h0 + b * waves * HPW + slot;
+      raw[b] = h < heads ? ntload(src + static_cast<int64_t>(h) * D)
+                         : make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  // The row and the norm weights are on their way while the angles are made.
+  load(wave * HPW);
+  const uint4 wq = *reinterpret_cast<const uint4*>(q_norm + 8 * j);
+  const uint4 wk = *reinterpret_cast<const uint4*>(k_norm + 8 * j);
+  const float pos = static_cast<float>(positions[row]);
+  for (int p = threadIdx.x; p < H2; p += blockDim.x) {
+    float sv, cv;
+    sincosf(pos * inv_freq[p], &sv, &cv);
+    s_cs[p] = bf16_to_f32(f32_to_bf16(cv));
+    s_sn[p] = bf16_to_f32(f32_to_bf16(sv));
+  }
+  __syncthreads();
+  // The sign of rotate_half goes into the sine (bf16r(-v) = -bf16r(v)).
   float cs[8], sn[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     cs[k] = s_cs[pair0 + k];
-    sn[k] = s_sn[pair0 + k];
+    sn[k] = lower ? -s_sn[pair0 + k] : s_sn[pair0 + k];
   }
-  const int heads = hq + 2 * hkv;
-  for (int h0 = wave * HPW; h0 < heads; h0 += waves * HPW) {
-    const int h = h0 + slot;
-    const bool live = h < heads;
-    const bool is_v = h >= hq + hkv;
-    const uint16_t* src = qkv + row * qkv_stride + static_cast<int64_t>(h) * D + 8 * j;
-    const uint4 raw = live ? *reinterpret_cast<const uint4*>(src) : make_uint4(0u, 0u, 0u, 0u);
-    const uint32_t rv[4] = {raw.x, raw.y, raw.z, raw.w};
-    float x[8];
+  for (int h0 = wave * HPW; h0 < heads;) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      x[2 * k] = bf16_to_f32(rv[k] & 0xffffu);
-      x[2 * k + 1] = bf16_to_f32(rv[k] >> 16);
-    }
-    // RMS over the head's D dims: the lane's 8 squares, then the head's lanes.
-    float ss = 0.0f;
+    for (int b = 0; b < kBatch; ++b) {
+      const int h = h0 + b * waves * HPW + slot;
+      const bool live = h < heads;
+      const bool is_v = h >= hq + hkv;
+      const uint32_t rv[4] = {raw[b].x, raw[b].y, raw[b].z, raw[b].w};
+      Pair x[4];
+      // RMS over the head's D dims: the lane's 8 squares, then the head's lanes.
+      float ss = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) ss += x[k] * x[k];
+      for (int k = 0; k < 4; ++k) {
+        x[k] = unpack(rv[k]);
+        ss += x[k].lo * x[k].lo;
+        ss += x[k].hi * x[k].hi;
+      }
 #pragma unroll
-    for (int d = LPH / 2; d >= 1; d >>= 1) ss += __shfl_xor(ss, d);
-    const float r = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
-    const uint16_t* w = (h < hq ? q_norm : k_norm) + 8 * j;
-    const uint4 wraw = (live && !is_v) ? *reinterpret_cast<const uint4*>(w)
-                                       : make_uint4(0u, 0u, 0u, 0u);
-    const uint32_t wv[4] = {wraw.x, wraw.y, wraw.z, wraw.w};
-    uint32_t nx[4];
+      for (int d = LPH / 2; d >= 1; d >>= 1) ss += __shfl_xor(ss, d);
+      const float r = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
+      const uint4 wraw = h < hq ? wq : wk;
+      const uint32_t wv[4] = {wraw.x, wraw.y, wraw.z, wraw.w};
+      uint32_t nx[4], ny[4], o[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float lo = bf16_to_f32(wv[k] & 0xffffu) * bf16r(x[2 * k] * r);
-      const float hi = bf16_to_f32(wv[k] >> 16) * bf16r(x[2 * k + 1] * r);
-      nx[k] = pack_bf16x2(lo, hi);
-    }
-    // The rotary partner's normed values (exact: bf16 pairs).
-    uint32_t ny[4];
+      for (int k = 0; k < 4; ++k) {
+        const Pair w = unpack(wv[k]);
+        const Pair n = bf16r(x[k].lo * r, x[k].hi * r);
+        nx[k] = pack_bf16x2(w.lo * n.lo, w.hi * n.hi);
+      }
+      // The rotary partner's normed values (exact: bf16 pairs).
 #pragma unroll
-    for (int k = 0; k < 4; ++k) ny[k] = __shfl_xor(nx[k], LPH / 2);
-    uint32_t o[4];
+      for (int k = 0; k < 4; ++k) ny[k] = __shfl_xor(nx[k], LPH / 2);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float e[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const float a = bf16_to_f32(t ? (nx[k] >> 16) : (nx[k] & 0xffffu));
-        const float b = bf16_to_f32(t ? (ny[k] >> 16) : (ny[k] & 0xffffu));
-        const int q = 2 * k + t;
+      for (int k = 0; k < 4; ++k) {
         // x*cos + rotate_half(x)*sin, rotate_half(x) = (-x2, x1), with the
         // rounding points of transformers' bf16 tensors: each product is
-        // rounded to bf16, then their sum (bf16r(-v) = -bf16r(v)).
-        const float ac = bf16r(a * cs[q]);
-        const float bs = bf16r(b * sn[q]);
-        e[t] = lower ? ac - bs : ac + bs;
+        // rounded to bf16, then their sum.
+        const Pair a = unpack(nx[k]), p = unpack(ny[k]);
+        const Pair ac = bf16r(a.lo * cs[2 * k], a.hi * cs[2 * k + 1]);
+        const Pair bs = bf16r(p.lo * sn[2 * k], p.hi * sn[2 * k + 1]);
+        o[k] = pack_bf16x2(ac.lo + bs.lo, ac.hi + bs.hi);
       }
-      o[k] = pack_bf16x2(e[0], e[1]);
+      if (!live) continue;
+      if (is_v) {
+        *reinterpret_cast<uint4*>(v_out + static_cast<int64_t>(h - hq - hkv) * kv_head_stride +
+                                  row * D + 8 * j) = raw[b];
+      } else {
+        uint16_t* dst = h < hq ? q_out + row * q_row_stride + static_cast<int64_t>(h) * D
+                               : k_out + static_cast<int64_t>(h - hq) * kv_head_stride + row * D;
+        *reinterpret_cast<uint4*>(dst + 8 * j) = make_uint4(o[0], o[1], o[2], o[3]);
+      }
     }
-    if (!live) continue;
-    if (is_v) {
-      *reinterpret_cast<uint4*>(v_out + static_cast<int64_t>(h - hq - hkv) * kv_head_stride +
-                                row * D + 8 * j) = raw;
-    } else {
-      uint16_t* dst = h < hq ? q_out + row * q_row_stride + static_cast<int64_t>(h) * D
-                             : k_out + static_cast<int64_t>(h - hq) * kv_head_stride + row * D;
-      *reinterpret_cast<uint4*>(dst + 8 * j) = make_uint4(o[0], o[1], o[2], o[3]);
-    }
+    h0 += kBatch * waves * HPW;
+    if (h0 < heads) load(h0);
   }
 }
 
 // out[r, i] = bf16(bf16(silu(gate[r, i])) * up[r, i]); gate = gu[r, :I],
-// up = gu[r, I:2I].  8 elements per thread.
+// up = gu[r, I:2I].  A workgroup takes kSiluChunks * 256 chunks of 8 elements
+// of one row (parts = workgroups per row), so that the row is one scalar
+// division and a thread has four loads in flight.
+constexpr int kSiluChunks = 2;
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gu,
                                                        int64_t gu_stride, int inter,
                                                        uint16_t* __restrict__ out,
-                                                       int64_t out_stride, int64_t chunks) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k >= chunks) return;
-  const int per_row = inter / 8;
-  const int64_t row = k / per_row;
-  const int e = 8 * static_cast<int>(k - row * per_row);
-  const uint4 g = *reinterpret_cast<const uint4*>(gu + row * gu_stride + e);
-  const uint4 u = *reinterpret_cast<const uint4*>(gu + row * gu_stride + inter + e);
-  const uint32_t gv[4] = {g.x, g.y, g.z, g.w};
-  const uint32_t uv[4] = {u.x, u.y, u.z, u.w};
-  uint32_t o[4];
+                                                       int64_t out_stride, uint32_t parts,
+                                                       int64_t items) {
+  for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+    const int64_t row = item / parts;
+    const uint32_t part = static_cast<uint32_t>(item - row * parts);
+    const uint32_t e0 = 8 * (part * kSiluChunks * 256 + threadIdx.x);
+    const uint16_t* gr = gu + row * gu_stride;
+    uint4 g[kSiluChunks], u[kSiluChunks];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    float v[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const float x = bf16_to_f32(h ? (gv[q] >> 16) : (gv[q] & 0xffffu));
-      const float up = bf16_to_f32(h ? (uv[q] >> 16) : (uv[q] & 0xffffu));
-      const float s = bf16r(x / (1.0f + expf(-x)));
-      v[h] = s * up;
+    for (int c = 0; c < kSiluChunks; ++c) {
+      const uint32_t e = e0 + c * 8 * 256;
+      const bool live = e < static_cast<uint32_t>(inter);
+      g[c] = live ? ntload(gr + e) : make_uint4(0u, 0u, 0u, 0u);
+      u[c] = live ? ntload(gr + inter + e) : make_uint4(0u, 0u, 0u, 0u);
     }
-    o[q] = pack_bf16x2(v[0], v[1]);
+#pragma unroll
+    for (int c = 0; c < kSiluChunks; ++c) {
+      const uint32_t e = e0 + c * 8 * 256;
+      if (e >= static_cast<uint32_t>(inter)) continue;
+      const uint32_t gv[4] = {g[c].x, g[c].y, g[c].z, g[c].w};
+      const uint32_t uv[4] = {u[c].x, u[c].y, u[c].z, u[c].w};
+      uint32_t o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const Pair x = unpack(gv[q]), up = unpack(uv[q]);
+        const Pair s = bf16r(x.lo / (1.0f + expf(-x.lo)), x.hi / (1.0f + expf(-x.hi)));
+        o[q] = pack_bf16x2(s.lo * up.lo, s.hi * up.hi);
+      }
+      *reinterpret_cast<uint4*>(out + row * out_stride + e) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
   }
-  *reinterpret_cast<uint4*>(out + row * out_stride + e) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
 // out[k, l*width .. (l+1)*width) = src_l[index[k], :width]; one workgroup per
@@ -302,12 +353,20 @@ extern "C" int sg_add_rmsnorm(const SgAddRmsNormArgs* args, sg_stream_t stream) 
                  (!a.residual_dev || aligned16(a.residual_dev)) &&
                  (!a.residual_out_dev || aligned16(a.residual_out_dev)),
              "tensors must be 16-byte aligned");
-  add_rmsnorm_kernel<<<dim3(a.num_rows), dim3(kNormThreads), 0,
-                       static_cast<hipStream_t>(stream)>>>(
-      static_cast<const uint16_t*>(a.x_dev), static_cast<const uint16_t*>(a.residual_dev),
-      static_cast<const uint16_t*>(a.weight_dev), static_cast<uint16_t*>(a.out_dev),
-      static_cast<uint16_t*>(a.residual_out_dev), a.hidden, a.x_stride, a.residual_stride,
-      a.out_stride, a.residual_out_stride, a.eps);
+  auto go = [&](auto kernel) {
+    kernel<<<dim3(a.num_rows), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<const uint16_t*>(a.x_dev), static_cast<const uint16_t*>(a.residual_dev),
+        static_cast<const uint16_t*>(a.weight_dev), static_cast<uint16_t*>(a.out_dev),
+        static_cast<uint16_t*>(a.residual_out_dev), a.hidden, a.x_stride, a.residual_stride,
+        a.out_stride, a.residual_out_stride, a.eps);
+  };
+  const bool res = a.residual_dev != nullptr;
+  switch ((a.hidden + 8 * kNormThreads - 1) / (8 * kNormThreads)) {
+    case 1: res ? go(add_rmsnorm_kernel<1, true>) : go(add_rmsnorm_kernel<1, false>); break;
+    case 2: res ? go(add_rmsnorm_kernel<2, true>) : go(add_rmsnorm_kernel<2, false>); break;
+    case 3: res ? go(add_rmsnorm_kernel<3, true>) : go(add_rmsnorm_kernel<3, false>); break;
+    default: res ? go(add_rmsnorm_kernel<4, true>) : go(add_rmsnorm_kernel<4, false>); break;
+  }
   SG_LAUNCH_CHECK();
   return SG_OK;
 }
@@ -367,13 +426,13 @@ extern "C" int sg_silu_mul(const void* gate_up_dev, int64_t gate_up_row_stride,
                  out_row_stride >= intermediate && (gate_up_row_stride | out_row_stride) % 8 == 0,
              "row strides must cover the rows and be multiples of 8");
   SG_REQUIRE(aligned16(gate_up_dev) && aligned16(out_dev), "tensors must be 16-byte aligned");
-  const int64_t chunks = static_cast<int64_t>(num_rows) * (intermediate / 8);
-  const int64_t blocks = (chunks + 255) / 256;
-  SG_REQUIRE(blocks < INT32_MAX, "too many rows");
-  silu_mul_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+  constexpr int kPart = 8 * 256 * kSiluChunks;  // elements of a workgroup's part of a row
+  const uint32_t parts = (static_cast<uint32_t>(intermediate) + kPart - 1) / kPart;
+  const int64_t items = static_cast<int64_t>(num_rows) * parts;
+  silu_mul_kernel<<<dim3(static_cast<unsigned>(std::min<int64_t>(items, 1 << 20))), dim3(256), 0,
                     static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(gate_up_dev), gate_up_row_stride, intermediate,
-      static_cast<uint16_t*>(out_dev), out_row_stride, chunks);
+      static_cast<uint16_t*>(out_dev), out_row_stride, parts, items);
   SG_LAUNCH_CHECK();
   return SG_OK;
 }

@@ -136,6 +136,59 @@ def test_silu_mul_and_feature_gather(device):
     assert int(bad.status.item()) == -1 and torch.equal(bad[1], torch.zeros_like(bad[1]))
 
 
+@pytest.mark.parametrize("rows,hidden", [(3, 8), (2, 2040), (2, 2048), (3, 2056), (2, 4104),
+                                         (1, 6144), (2, 6152), (2, 8192)])
+def test_add_rmsnorm_at_the_chunk_edges(device, rows, hidden):
+    from specgrove_amd import target
+    g = torch.Generator().manual_seed(hidden)
+    wide = torch.randn((rows, hidden + 24), generator=g).to(torch.bfloat16).to(device)
+    x, res = wide[:, 8:8 + hidden], torch.randn((rows, hidden), generator=g).to(wide)
+    w = (1 + 0.1 * torch.randn(hidden, generator=g)).to(wide)
+    for r in (None, res):
+        want_sum = x if r is None else x + r
+        f = want_sum.float()
+        normed = (f * torch.rsqrt(f.square().mean(1, keepdim=True) + 1e-6)).to(torch.bfloat16)
+        out, total = target.add_rmsnorm(x, w, 1e-6, r, want_sum=True)
+        assert torch.equal(total, want_sum)
+        _close_bf16(out, normed * w, f"rmsnorm {rows}x{hidden}")
+
+
+@pytest.mark.parametrize("rows,inter", [(3, 8), (5, 2048), (2, 2056), (3, 4088), (2, 4096),
+                                        (3, 4104), (2, 9728), (70000, 8)])
+def test_silu_mul_at_the_part_edges(device, rows, inter):
+    from specgrove_amd import target
+    g = torch.Generator().manual_seed(inter)
+    gu = (torch.randn((rows, 2 * inter), generator=g) * 3).to(torch.bfloat16).to(device)
+    _close_bf16(target.silu_mul(gu), torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:],
+                f"silu*up {rows}x{inter}")
+
+
+@pytest.mark.parametrize("dim,hq,hkv", [(128, 1, 1), (128, 47, 1), (128, 64, 8), (128, 16, 16),
+                                        (64, 32, 32), (64, 96, 3), (64, 128, 16)])
+def test_qk_norm_rope_over_head_counts(device, dim, hq, hkv):
+    # Heads of one load batch, of one more than a batch, and of several.
+    from specgrove_amd import target
+    rows = 5
+    g = torch.Generator().manual_seed(hq + dim)
+    qkv = torch.randn((rows, (hq + 2 * hkv) * dim), generator=g).to(torch.bfloat16).to(device)
+    qn, kn = ((1 + 0.2 * torch.randn(dim, generator=g)).to(qkv) for _ in range(2))
+    inv = (1.0 / (1e6 ** (torch.arange(0, dim, 2).float() / dim))).to(device)
+    pos = torch.tensor([0, 1, 63, 4097, 32767], device=device)
+    x = qkv.view(rows, hq + 2 * hkv, dim)
+    w = torch.cat([qn.expand(hq, dim), kn.expand(hkv, dim)])
+    f = x[:, :hq + hkv].float()
+    n = (f * torch.rsqrt(f.square().mean(2, keepdim=True) + 1e-6)).to(torch.bfloat16) * w
+    angle = pos.float()[:, None] * inv
+    cos, sin = (torch.cat([t, t], 1).to(torch.bfloat16)[:, None] for t in (angle.cos(),
+                                                                           angle.sin()))
+    half = torch.cat([-n[..., dim // 2:], n[..., :dim // 2]], 2)
+    want = n * cos + half * sin
+    q, k, v = target.qk_norm_rope(qkv, hq, hkv, dim, qn, kn, inv, pos, 1e-6)
+    _close_rotary(q, want[:, :hq], "q")
+    _close_rotary(k.transpose(0, 1), want[:, hq:], "k")
+    assert torch.equal(v.transpose(0, 1), x[:, hq + hkv:])
+
+
 def _tiny_models(transformers, device):
     from specgrove_amd import attention
     from specgrove_amd.target import Qwen3TargetStack
