@@ -26,6 +26,7 @@ tree K/V.
 from __future__ import annotations
 
 from dataclasses import dataclass, field
+from itertools import chain
 from typing import Sequence
 
 import numpy as np
@@ -49,6 +50,7 @@ class PackedTreeMask:
     row_offset_host: np.ndarray
     prefix_len_host: np.ndarray
     plans: dict = field(default_factory=dict)
+    streams: set = field(default_factory=set)  # handles of the streams that ordered the copies
 
     @property
     def num_rows(self) -> int:
@@ -61,8 +63,42 @@ class PackedTreeMask:
         if key not in self.plans:
             self.plans[key] = ops.plan_attention(
                 self.row_offset_host, self.prefix_len_host, num_q_heads, num_kv_heads,
-                head_dim).to(self.row_offset.device)
+                head_dim).to(self.row_offset.device, non_blocking=True)
+            self._ordered_here()
+        self._join()
         return self.plans[key]
+
+    def _ordered_here(self) -> None:
+        """The current stream ordered a copy of this mask."""
+        if self.row_offset.is_cuda:
+            self.streams.add(ops._stream_handle())
+
+    def _join(self) -> None:
+        """The mask's copies are ordered by the streams that were current when
+        it and its plans were made; any other stream waits for those first."""
+        if not self.streams:
+            return
+        here = ops._stream_handle()
+        for handle in self.streams:
+            if handle != here:
+                device = self.row_offset.device
+                torch.cuda.current_stream(device).wait_stream(
+                    torch.cuda.ExternalStream(handle, device=device) if handle
+                    else torch.cuda.default_stream(device))
+
+
+def _parents_precede(flat: np.ndarray, row_offset: np.ndarray, parents_list) -> bool:
+    """Whether every tree has its root (-1) first and every parent before its
+    children; ``flat`` holds the trees' parents end to end."""
+    if flat.size == 0:
+        return True
+    if flat.dtype.kind not in "iu":
+        return all(p[0] == -1 and all(0 <= q < k for k, q in enumerate(p[1:], 1))
+                   for p in parents_list)
+    rows = np.diff(row_offset)
+    local = np.arange(flat.size) - np.repeat(row_offset[:-1], rows)
+    root = local == 0
+    return bool(np.where(root, flat == -1, (flat >= 0) & (flat < local)).all())
 
 
 def build_tree_mask(pool, caches: Sequence, parents_list: Sequence[Sequence[int]],
@@ -76,11 +112,10 @@ def build_tree_mask(pool, caches: Sequence, parents_list: Sequence[Sequence[int]
     rows = [len(p) for p in parents_list]
     row_offset = np.zeros(len(rows) + 1, np.int32)
     np.cumsum(rows, out=row_offset[1:])
-    parent = np.concatenate([np.asarray(p, np.int32) for p in parents_list]) if rows else \
-        np.zeros(0, np.int32)
-    for p in parents_list:
-        if len(p) == 0 or p[0] != -1 or any(not 0 <= q < k for k, q in enumerate(p[1:], 1)):
-            raise ValueError("Tree parents must precede their children")
+    flat = np.asarray(list(chain.from_iterable(parents_list)))
+    if 0 in rows or not _parents_precede(flat, row_offset, parents_list):
+        raise ValueError("Tree parents must precede their children")
+    parent = flat.astype(np.int32)
     if prefix_start is None:
         prefix_len = np.asarray([pool.lengths[c.slot] for c in caches], np.int32)
         prefix_start = np.asarray([c.slot * pool.capacity for c in caches], np.int64)
@@ -95,9 +130,9 @@ def build_tree_mask(pool, caches: Sequence, parents_list: Sequence[Sequence[int]
     if words32.size % 2:
         words32 = np.concatenate([words32, np.zeros(1, np.int32)])
     host = np.concatenate([prefix_start.astype(np.int64), words32.view(np.int64)])
-    meta = torch.from_numpy(host).to(dev)
+    meta = ops.upload(host, dev)
     meta32 = meta[n:].view(torch.int32)
-    return PackedTreeMask(
+    mask = PackedTreeMask(
         pool=pool,
         row_offset=meta32[:n + 1],
         parent=meta32[2 * n + 1:2 * n + 1 + parent.size],
@@ -106,6 +141,8 @@ def build_tree_mask(pool, caches: Sequence, parents_list: Sequence[Sequence[int]
         row_offset_host=row_offset,
         prefix_len_host=prefix_len,
     )
+    mask._ordered_here()
+    return mask
 
 
 def pack_block_inputs(states, blocks, cache_lengths: Sequence[int],

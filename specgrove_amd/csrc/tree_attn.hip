@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstring>
+#include <functional>
 #include <numeric>
 #include <queue>
 #include <type_traits>
@@ -1181,17 +1182,27 @@ extern "C" int sg_tree_attn_plan(int32_t num_requests, const int32_t* row_offset
   // dispatcher places workgroup b on XCD b % 8, whose L2 then serves the
   // re-reads.  (A placement heuristic only.)
   std::vector<int64_t> xcd_of(static_cast<size_t>(num_requests) * num_kv_heads, -1);
+  // The least loaded list (the first of equals) of each XCD's lists, or of all
+  // where there are fewer lists than XCDs, is the top of a heap: scanning the
+  // lists for every unit took half of a plan's time.
+  const int64_t classes = bins >= kXcds ? kXcds : 1;
+  using Entry = std::pair<int64_t, int64_t>;  // (load, list)
+  std::vector<std::priority_queue<Entry, std::vector<Entry>, std::greater<Entry>>> least(classes);
+  for (int64_t b = 0; b < bins; ++b) least[b % classes].push({0, b});
   for (size_t k : order) {
     const size_t key = static_cast<size_t>(units[k].req) * num_kv_heads + units[k].kv_head;
-    int64_t b = -1;
-    if (xcd_of[key] >= 0 && bins >= kXcds) {
-      for (int64_t c = xcd_of[key]; c < bins; c += kXcds)
-        if (b < 0 || load[c] < load[b]) b = c;
+    int64_t cls = 0;
+    if (xcd_of[key] >= 0 && classes > 1) {
+      cls = xcd_of[key];
     } else {
-      b = std::min_element(load.begin(), load.end()) - load.begin();
-      xcd_of[key] = b % kXcds;
+      for (int64_t c = 1; c < classes; ++c)
+        if (least[c].top() < least[cls].top()) cls = c;
+      xcd_of[key] = least[cls].top().second % kXcds;
     }
+    const int64_t b = least[cls].top().second;
+    least[cls].pop();
     load[b] += cost[k];
+    least[cls].push({load[b], b});
     bin_units[b].push_back(k);
   }
   // Local search: move a unit out of the most loaded list, or swap it with a

@@ -63,6 +63,16 @@ class PreparedCall:
         return self
 
 
+def upload(array: np.ndarray, device) -> torch.Tensor:
+    """A host array on the device, copied in stream order from pinned memory:
+    the host does not wait for the stream's earlier work.  (While a stream is
+    captured the copy is a plain one, which capture refuses.)"""
+    host = torch.from_numpy(array)
+    if torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return host.to(device)
+    return host.pin_memory().to(device, non_blocking=True)
+
+
 def _require(cond: bool, message: str) -> None:
     if not cond:
         raise ValueError(message)
@@ -128,14 +138,19 @@ class AttnPlan:
     def num_rows(self) -> int:
         return int(self.header[9])
 
-    def to(self, device) -> "AttnPlan":
+    def to(self, device, non_blocking: bool = False) -> "AttnPlan":
         """Copy the plan to the device and allocate its workspace (the fp32
         partial results of split units; every slot is written before the merge
-        kernel reads it, so its initial contents do not matter)."""
-        self.device = torch.from_numpy(self.host).to(device, non_blocking=False)
+        kernel reads it, so its initial contents do not matter).  With
+        ``non_blocking`` the copy is only ordered on the current stream."""
+        self.device = upload(self.host, device) if non_blocking else \
+            torch.from_numpy(self.host).to(device, non_blocking=False)
         self.workspace = torch.zeros(max(self.workspace_bytes, 16), dtype=torch.uint8,
                                      device=device)
         return self
+
+
+_PLAN_BYTES = 1 << 16  # about 1,300 units
 
 
 def plan_attention(row_offset, prefix_len, num_q_heads: int, num_kv_heads: int,
@@ -152,14 +167,18 @@ def plan_attention(row_offset, prefix_len, num_q_heads: int, num_kv_heads: int,
     ws = ctypes.c_size_t()
     args = (n, ro.ctypes.data_as(i32p), pl.ctypes.data_as(i32p), num_q_heads,
             num_kv_heads, head_dim, target_units)
-    _lib.check(lib.sg_tree_attn_plan(*args, None, 0, ctypes.byref(plan_bytes),
-                                     ctypes.byref(units), ctypes.byref(merges),
-                                     ctypes.byref(ws)), "sg_tree_attn_plan")
-    host = np.zeros(plan_bytes.value, dtype=np.uint8)
-    _lib.check(lib.sg_tree_attn_plan(*args, host.ctypes.data_as(ctypes.c_void_p),
-                                     host.nbytes, ctypes.byref(plan_bytes),
-                                     ctypes.byref(units), ctypes.byref(merges),
-                                     ctypes.byref(ws)), "sg_tree_attn_plan")
+    # The plan is made once, into a buffer that holds most plans; the size it
+    # reports serves a larger one.
+    host = np.zeros(_PLAN_BYTES, dtype=np.uint8)
+    for _ in range(2):
+        rc = lib.sg_tree_attn_plan(*args, host.ctypes.data_as(ctypes.c_void_p), host.nbytes,
+                                   ctypes.byref(plan_bytes), ctypes.byref(units),
+                                   ctypes.byref(merges), ctypes.byref(ws))
+        if rc == 0 or plan_bytes.value <= host.nbytes:
+            break
+        host = np.zeros(plan_bytes.value, dtype=np.uint8)
+    _lib.check(rc, "sg_tree_attn_plan")
+    host = host[:plan_bytes.value].copy()
     return AttnPlan(host, units.value, merges.value, ws.value, num_q_heads,
                     num_kv_heads, head_dim)
 

@@ -219,7 +219,6 @@ class Qwen3TargetStack:
             raise ValueError("Packed rows disagree with the tree mask")
         positions = position_ids.reshape(-1).to(torch.int64).contiguous()
         hq, hkv, d = self.num_q_heads, self.num_kv_heads, self.head_dim
-        plan = mask.plan(hq, hkv, d)
         x = torch.nn.functional.embedding(input_ids[0], self.embed)
         states = [x] if output_hidden_states else None
         residual = None
@@ -229,6 +228,8 @@ class Qwen3TargetStack:
             if states is not None and index > 0:
                 states.append(residual)
             qkv = torch.matmul(h, layer.wqkv.T)
+            if index == 0:  # made while the GPU runs what is launched so far
+                plan = mask.plan(hq, hkv, d)
             q, k, v = qk_norm_rope(qkv, hq, hkv, d, layer.q_norm, layer.k_norm, self.inv_freq,
                                    positions, self.eps)
             k_new, v_new = cache.update(k[None], v[None], index)

@@ -99,6 +99,20 @@ def test_plan_covers_every_row_and_key_once(target):
     _check_plan(W.tiny_attention_workload(), target)
 
 
+@pytest.mark.parametrize("requests,heads", [(1, 1), (160, 8), (170, 8), (300, 16)])
+def test_plans_around_the_first_buffer_are_whole(requests, heads):
+    # 1,280 units fit the buffer a plan is first made into, 1,360 do not.
+    wl = W.AttentionWorkload("sizes", 4 * heads, heads, 128,
+                             np.arange(requests, dtype=np.int32) % 97 + 300,
+                             [[-1]] * requests, [[]] * requests, 448)
+    plan = ops.plan_attention(wl.row_offset, wl.prefix_len, 4 * heads, heads, 128)
+    _, units, merges, bins = ops.decode_plan(plan)
+    assert plan.host.nbytes == 64 + units.nbytes + merges.nbytes + bins.nbytes
+    assert int(bins[-1]) == len(units) >= requests * heads
+    seen = {(int(u[0]), int(u[1])) for u in units}
+    assert seen == {(i, g) for i in range(requests) for g in range(heads)}
+
+
 def test_plan_rejects_oversized_trees_and_bad_heads():
     with pytest.raises(ValueError):
         ops.plan_attention([0, 300], [10], 32, 8, 128)

@@ -312,6 +312,36 @@ def test_stack_matches_transformers_on_a_packed_wave(device):
     assert len(got.hidden_states) == 3 and torch.equal(got.hidden_states[2], got.last_hidden_state)
 
 
+@pytest.mark.parametrize("planned_here", [True, False])
+def test_a_mask_used_on_another_stream_waits_for_its_copies(device, planned_here):
+    from types import SimpleNamespace
+    from specgrove_amd import attention
+    lengths, tree = [300, 517, 64], [-1, 0, 1, 1, 0]
+    pool = SimpleNamespace(lengths=lengths, capacity=576)
+    caches = [SimpleNamespace(slot=i) for i in range(3)]
+    g = torch.Generator(device).manual_seed(1)
+    pool.key_storage = [torch.randn((2, 3 * 576, 64), generator=g, device=device).to(torch.bfloat16)]
+    pool.value_storage = [torch.randn_like(pool.key_storage[0])]
+    q, k, v = (torch.randn((1, h, 15, 64), generator=g, device=device).to(torch.bfloat16)
+               for h in (4, 2, 2))
+    module = SimpleNamespace(layer_idx=0)
+    want = attention.tree_attention_forward(
+        module, q, k, v, attention.build_tree_mask(pool, caches, [tree] * 3, device))[0]
+    busy = torch.randn((4096, 4096), device=device)
+    torch.cuda.synchronize()
+    for _ in range(20):  # the copies queue up behind these
+        busy = busy @ busy * 1e-3
+    mask = attention.build_tree_mask(pool, caches, [tree] * 3, device)
+    if planned_here:
+        mask.plan(4, 2, 64)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        got = attention.tree_attention_forward(module, q, k, v, mask)[0]
+    side.synchronize()
+    assert torch.equal(got, want)
+    torch.cuda.synchronize()
+
+
 def test_decode_loop_runs_on_the_stack(device):
     transformers = pytest.importorskip("transformers")
     from specgrove_amd import decode, scheduler

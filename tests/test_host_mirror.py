@@ -106,6 +106,35 @@ def test_packed_inputs_reject_bad_trees_and_foreign_pools():
         attention.pack_block_inputs(states, blocks, [5, 6], [0, 5], 11, torch.bfloat16, "cpu")
 
 
+@pytest.mark.parametrize("kind", ["list", "int32", "int64", "float", "mixed"])
+def test_tree_checks_over_whole_waves_agree_with_each_tree_alone(kind):
+    rng = np.random.default_rng(len(kind))
+
+    def form(p, k):
+        if kind == "list" or (kind == "mixed" and k % 2):
+            return p
+        return np.asarray(p, kind if kind != "mixed" else "int64")
+
+    for _ in range(300):
+        trees = []
+        for k in range(int(rng.integers(1, 5))):
+            p = [-1] + [int(rng.integers(0, n)) for n in range(1, int(rng.integers(1, 40)))]
+            if rng.random() < 0.3:
+                p[int(rng.integers(0, len(p)))] = int(rng.integers(-3, len(p) + 2))
+            trees.append(form([] if rng.random() < 0.02 else p, k))
+        good = all(len(p) > 0 and p[0] == -1 and all(0 <= q < n for n, q in enumerate(p[1:], 1))
+                   for p in trees)
+        pool = SimpleNamespace(lengths=[7] * len(trees), capacity=64)
+        caches = [SimpleNamespace(slot=i) for i in range(len(trees))]
+        if not good:
+            with pytest.raises(ValueError, match="precede"):
+                attention.build_tree_mask(pool, caches, trees, "cpu")
+            continue
+        mask = attention.build_tree_mask(pool, caches, trees, "cpu")
+        assert mask.parent.tolist() == [int(q) for p in trees for q in p]
+        assert mask.row_offset.tolist() == [0] + np.cumsum([len(p) for p in trees]).tolist()
+
+
 def test_tree_cache_records_new_rows_and_commit_checks():
     pool, _ = _pool([5, 60])
     packed, lengths, offsets, total = pack_cache_sequence(pool.caches)
