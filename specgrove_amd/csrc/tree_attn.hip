@@ -51,12 +51,22 @@ typedef __attribute__((ext_vector_type(4))) short short4_t;
 typedef __attribute__((ext_vector_type(8))) short short8_t;
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 
-constexpr int kThreads = 256;
 constexpr int kQPerUnit = 128;
 constexpr int kTileKeys = 32;                   // keys per tile: one 32-key MFMA block
 constexpr int kListsPerCU = 2;                  // resident workgroups per CU
-constexpr int kStages = 4;
-constexpr int kWaves = 4;
+// Shape of a workgroup.  kSmall: launches of at most one workgroup per CU at
+// D = 128, where a workgroup has all of its CU: eight waves (two key streams for
+// four q-groups, so two waves per matrix unit) and copies three windows ahead
+// (137 KB of LDS).  16 requests, 512 rows, 354-2,036 cached tokens, 32 q / 8 kv
+// heads: 38.3 -> 36.5 us (37.1 us one window ahead; 43.4 us with four waves).
+// D = 64 measured equal and keeps four waves.
+template <bool kSmall>
+struct Shape {
+  static constexpr int kWaves = kSmall ? 8 : 4;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int kAhead = kSmall ? 3 : 1;   // windows from a copy to its use
+  static constexpr int kStages = 2 * kAhead + 2;  // tiles in each ring
+};
 constexpr int kMaxTreeRows = 256;
 constexpr int kAncWords = kMaxTreeRows / 32;
 constexpr int kMergeThreads = 256;
@@ -267,13 +277,13 @@ __device__ void poison_unit(const SgTreeAttnArgs& a, const AttnUnit& u, int r0) 
   const float qnan = __builtin_nanf("");
   if (u.partial >= 0) {
     float* part = static_cast<float*>(a.workspace_dev) + partial_floats(D) * u.partial;
-    for (int k = tid; k < static_cast<int>(partial_floats(D)); k += kThreads)
+    for (int k = tid; k < static_cast<int>(partial_floats(D)); k += blockDim.x)
       part[k] = (k >= kQPerUnit * D && k < kQPerUnit * (D + 1)) ? 0.0f : qnan;
     return;
   }
   const int G = a.num_q_heads / a.num_kv_heads;
   uint16_t* out = static_cast<uint16_t*>(a.out_dev);
-  for (int k = tid; k < u.row_count * G * D; k += kThreads) {
+  for (int k = tid; k < u.row_count * G * D; k += blockDim.x) {
     const int rr = k / (G * D);
     const int h = (k / D) % G;
     const int64_t row = static_cast<int64_t>(r0) + u.row_begin + rr;
@@ -284,8 +294,12 @@ __device__ void poison_unit(const SgTreeAttnArgs& a, const AttnUnit& u, int r0) 
 }
 
 // Attention of one work unit by the whole workgroup.
-template <int D>
+template <int D, bool kSmall>
 __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUnit& u) {
+  constexpr int kWaves = Shape<kSmall>::kWaves;
+  constexpr int kThreads = Shape<kSmall>::kThreads;
+  constexpr int kAhead = Shape<kSmall>::kAhead;
+  constexpr int kStages = Shape<kSmall>::kStages;
   constexpr int KB = D / 16;                     // QK^T k-blocks of 16 head dims
   constexpr int DB = D / 32;                     // PV blocks of 32 head dims
   constexpr int ROWB = D * 2;                    // bytes per unpadded K/V row
@@ -295,9 +309,8 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   constexpr int DMAS = STAGEB / 1024 / kWaves;   // DMAs per wave per K (or V) tile
   constexpr int STATE = 2 + 16 * DB;             // floats per lane of a WaveState
   static_assert(DMAS >= 1, "tile too small for the workgroup");
-  static_assert(kStages == 4, "the issue schedule assumes a 4-tile ring");
   static_assert(kStages * STAGEB <= 65536, "ring offsets must fit the LDS immediate");
-  static_assert(2 * ((kStages * STAGEB) / (STATE * 64 * 4)) >= 2, "merge scratch");
+  static_assert(2 * ((kStages * STAGEB) / (STATE * 64 * 4)) >= kWaves / 2, "merge scratch");
   // Rings of kStages tiles of K and of V; reused as the merge scratch at the end.
   __shared__ __align__(1024) unsigned char s_k[kStages * STAGEB];
   __shared__ __align__(1024) unsigned char s_v[kStages * STAGEB];
@@ -312,12 +325,13 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   const int col = lane & 31;
   const int nq = (u.row_count * G + 31) / 32;   // q-groups in use, 1..4
   // Every window (one barrier) consumes two consecutive 32-key tiles.  With
-  // 1-2 q-groups two waves share a q-group ("key streams") and take one tile
+  // 1-2 q-groups (1-4 in eight waves) two waves share a q-group ("key streams") and take one tile
   // each; their results are merged at the end of the unit.  With 3-4 q-groups
   // every wave takes both tiles, one after the other.  Waves beyond
-  // nq*streams repeat stream 0's work on the same LDS data and discard it.
-  const int streams = nq <= 2 ? 2 : 1;
-  const bool both = streams == 1;
+  // nq*streams repeat stream 0's work on the same LDS data and discard it (in
+  // the small form they only copy).
+  const int streams = 2 * nq <= kWaves ? 2 : 1;
+  const bool both = !kSmall && streams == 1;
   const int qg = wave % nq;
   const int ks = wave / nq;                     // key stream of this wave
   const bool active = ks < streams;
@@ -357,8 +371,8 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   // With the tree tiles that a row tile cannot see left out (below), eight
   // 256-row chunks at 483-3,006 cached tokens (32 q / 8 kv heads): 138 -> 110 us.
   if (do_tree) {
-    {
-      // One node per thread (n <= kMaxTreeRows = kThreads).
+    if (tid < kMaxTreeRows) {
+      // One node per thread (n <= kMaxTreeRows <= kThreads).
       const int p = tid < n ? a.parent_dev[r0 + tid] : -1;
       const uint64_t linked = __ballot(lane > 0 && p == tid - 1);
       // The run starts at the highest unlinked lane at or below this one.
@@ -467,30 +481,49 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   // the PV products of those tiles and the QK products one block ahead, so
   // that the QK MFMAs overlap the softmax VALU work.  The QK products of
   // window i read the next group's tiles 2i+2, 2i+3 (two key streams) or
-  // tiles 2i+1, 2i+2 (one stream).  Window j issues V tiles 2j+2, 2j+3 and K
-  // tiles 2j+koff, 2j+koff+1 (koff 4, or 3 for one stream) into the ring
-  // slots that window j-1 finished reading; window i needs everything window
-  // i-1 issued, so nothing is in flight at its barrier.
+  // tiles 2i+1, 2i+2 (one stream).  Window j issues V tiles 2j+2A, 2j+2A+1
+  // (A = kAhead) and K tiles 2j+koff+2A-2, +1 (koff 4, or 3 for one stream)
+  // into the ring slots that window j-1 finished reading; window i needs
+  // everything that windows up to i-A issued, so what the A-1 windows in
+  // between issued may be in flight at its barrier.
   const int groups = (tiles + 1) / 2;
   const int koff = both ? 3 : 4;
   auto issue = [&](int j) {
     for (int k = 0; k < 2; ++k) {
-      const int t = 2 * j + 2 + k;
+      const int t = 2 * (j + kAhead) + k;
       if (t >= 0 && t < tiles) load_half(t, true);
     }
     for (int k = 0; k < 2; ++k) {
-      const int t = 2 * j + koff + k;
+      const int t = 2 * (j + kAhead - 1) + koff + k;
       if (t >= 0 && t < tiles) load_half(t, false);
     }
   };
-  // Wait until at most `newer` half tiles (the newest ones) are in flight.
-  auto wait_halves = [&](int newer) {
+  // Half tiles that window j issues.
+  auto issued = [&](int j) {
+    const int v = 2 * (j + kAhead), k = 2 * (j + kAhead - 1) + koff;
+    return (v >= 0 && v < tiles) + (v + 1 >= 0 && v + 1 < tiles) + (k >= 0 && k < tiles) +
+           (k + 1 >= 0 && k + 1 < tiles);
+  };
+  // Wait until only what windows first .. last issued is in flight.
+  auto wait_issued = [&](int first, int last) {
+    int newer = 0;
+    for (int j = first; j <= last; ++j) newer += issued(j);
     switch (newer) {
-      case 0: __builtin_amdgcn_s_waitcnt(vmcnt_encoding(0)); break;
-      case 1: __builtin_amdgcn_s_waitcnt(vmcnt_encoding(DMAS)); break;
-      case 2: __builtin_amdgcn_s_waitcnt(vmcnt_encoding(2 * DMAS)); break;
-      case 3: __builtin_amdgcn_s_waitcnt(vmcnt_encoding(3 * DMAS)); break;
-      default: __builtin_amdgcn_s_waitcnt(vmcnt_encoding(4 * DMAS)); break;
+#define SG_WAIT_CASE(n) \
+  case n: __builtin_amdgcn_s_waitcnt(vmcnt_encoding((n) * DMAS)); break;
+      SG_WAIT_CASE(1) SG_WAIT_CASE(2) SG_WAIT_CASE(3) SG_WAIT_CASE(4) SG_WAIT_CASE(5)
+      SG_WAIT_CASE(6) SG_WAIT_CASE(7) SG_WAIT_CASE(8) SG_WAIT_CASE(9) SG_WAIT_CASE(10)
+      SG_WAIT_CASE(11) SG_WAIT_CASE(12)
+#undef SG_WAIT_CASE
+      default: __builtin_amdgcn_s_waitcnt(vmcnt_encoding(0)); break;
+    }
+  };
+  // Window i's wait: constant while every window before it issued four halves.
+  auto wait_window = [&](int i) {
+    if (kAhead == 1 || 2 * (i + kAhead - 2) + koff + 1 < tiles) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_encoding(4 * (kAhead - 1) * DMAS));
+    } else {
+      wait_issued(i - kAhead + 1, i - 1);
     }
   };
 
@@ -606,31 +639,32 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
     }
   };
 
-  // Prologue: windows -2 and -1 of the issue schedule, then the first QK
-  // products, which need the K tiles of window -2; V tiles 0, 1 and K tiles
-  // koff-2, koff-1 of window -1 may still be in flight.
-  issue(-2);
-  issue(-1);
-  wait_halves((0 < tiles) + (1 < tiles) + (koff - 2 < tiles) + (koff - 1 < tiles));
+  // Prologue: the windows before the first of the issue schedule, then the
+  // first QK products, which need the K tiles of the first of them.  (Copies
+  // issued before the tree and Q are read: 1-3 % slower with two workgroups
+  // per CU, 42.7 instead of 36.5 us in the small form.)
+#pragma unroll
+  for (int j = -kAhead - 1; j < 0; ++j) issue(j);
+  wait_issued(-kAhead, -1);
   __syncthreads();
   floatx16 s_next;
 #pragma unroll
   for (int r = 0; r < 16; ++r) s_next[r] = 0.0f;
-  if (my_tile < tiles) s_next = qk(0);
+  if ((!kSmall || active) && my_tile < tiles) s_next = qk(0);
 
   // Windows whose issued tiles are all full prefix tiles (i < fast_end) need
   // none of the schedule arithmetic: the ring stages are compile-time and the
   // sources are one multiply away.
-  const int fast_end = (tiles_full - koff) / 2;
+  const int fast_end = (tiles_full - koff - 2 * kAhead + 2) / 2;
   const int64_t tile_bytes = static_cast<int64_t>(kTileKeys) * cstride * 2;
   const uint32_t k_lds_wave = lds_addr(s_k) + wave * DMAS * 1024;
   const uint32_t v_lds_wave = lds_addr(s_v) + wave * DMAS * 1024;
-  auto fast_issue = [&](int i, auto koff_tag, auto cur_tag, auto stream_tag) {
-    constexpr int kK = decltype(koff_tag)::value;
-    constexpr int kCur = decltype(cur_tag)::value;  // ring stage of tile 2i
+  // cur: ring stage of tile 2i.
+  auto fast_issue = [&](int i, auto koff_tag, int cur, auto stream_tag) {
+    constexpr int kK = decltype(koff_tag)::value + 2 * kAhead - 2;
     constexpr bool kStream = decltype(stream_tag)::value;
     const unsigned char* vb = reinterpret_cast<const unsigned char*>(vc) +
-                              static_cast<int64_t>(2 * i + 2) * tile_bytes;
+                              static_cast<int64_t>(2 * i + 2 * kAhead) * tile_bytes;
     const unsigned char* kb = reinterpret_cast<const unsigned char*>(kc) +
                               static_cast<int64_t>(2 * i + kK) * tile_bytes;
 #pragma unroll
@@ -638,21 +672,21 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
 #pragma unroll
       for (int d = 0; d < DMAS; ++d)
         dma16<kStream>(vb + k * tile_bytes, v_dma[d],
-                       v_lds_wave + ((kCur + 2 + k) % kStages) * STAGEB + 1024 * d);
+                       v_lds_wave + ((cur + 2 * kAhead + k) % kStages) * STAGEB + 1024 * d);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
 #pragma unroll
       for (int d = 0; d < DMAS; ++d)
         dma16<kStream>(kb + k * tile_bytes, k_dma[d],
-                       k_lds_wave + ((kCur + kK + k) % kStages) * STAGEB + 1024 * d);
+                       k_lds_wave + ((cur + kK + k) % kStages) * STAGEB + 1024 * d);
     }
   };
-  auto open_window = [&](int i, auto koff_tag, auto cur_tag, auto stream_tag) {
-    wait_halves(0);
+  auto open_window = [&](int i, auto koff_tag, int cur, auto stream_tag) {
+    wait_window(i);
     __syncthreads();
     if (i < fast_end) {
-      fast_issue(i, koff_tag, cur_tag, stream_tag);
+      fast_issue(i, koff_tag, cur, stream_tag);
     } else {
       issue(i);
     }
@@ -682,10 +716,26 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   const int steady_end = max(0, (tiles_full - koff + 2) / 2);
   int i = 0;
   bf16x8 pf[2];
-  if (both) {
+  if constexpr (kSmall) {
+    // Ring stages at run time: no window is left over for the slower loop below.
+    auto run = [&](auto stream_tag) {
+      for (; i < steady_end; ++i) {
+        const int cur = (2 * i) % kStages;
+        open_window(i, IntTag<4>{}, cur, stream_tag);
+        if (!active) continue;
+        softmax_qk((cur + 2) % kStages, pf);
+        pv(pf, cur);
+      }
+    };
+    if (stream_kv) {
+      run(BoolTag<true>{});
+    } else {
+      run(BoolTag<false>{});
+    }
+  } else if (both) {
     auto step = [&](int w, auto cur_tag, auto stream_tag) {
       constexpr int kCur = decltype(cur_tag)::value;
-      open_window(w, IntTag<3>{}, cur_tag, stream_tag);
+      open_window(w, IntTag<3>{}, kCur, stream_tag);
       softmax_qk(kCur + 1, pf);
       pv(pf, kCur);
       softmax_qk((kCur + 2) % kStages, pf);
@@ -707,7 +757,7 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
     // tile, so the unit is its K/V's only reader.
     auto step = [&](int w, auto cur_tag) {
       constexpr int kCur = decltype(cur_tag)::value;
-      open_window(w, IntTag<4>{}, cur_tag, BoolTag<true>{});
+      open_window(w, IntTag<4>{}, kCur, BoolTag<true>{});
       softmax_qk((kCur + 2) % kStages, pf);
       pv(pf, kCur);
     };
@@ -719,9 +769,10 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   // Remaining windows: runtime stages, masks from the key limit and the
   // ancestor bitsets.
   for (; i < groups; ++i) {
-    wait_halves(0);
+    wait_window(i);
     __syncthreads();
     issue(i);
+    if (kSmall && !active) continue;
     for (int b = 0; b < (both ? 2 : 1); ++b) {
       const int t = 2 * i + my_tile + b;
       const int t_next = both ? t + 1 : t + 2;
@@ -821,8 +872,16 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   static_assert(kSlotBytes + 32 * kPitch <= kStages * STAGEB &&
                     2 * 32 * kPitch <= kStages * STAGEB,
                 "output staging must fit the rings");
-  unsigned char* stage =
-      ((qg & 1) ? s_v : s_k) + (streams > 1 ? kSlotBytes : (qg >> 1) * 32 * kPitch);
+  unsigned char* stage;
+  if constexpr (kSmall) {
+    // The merge slots fill s_k (three of them) and the first of s_v.
+    static_assert(!kSmall || (kStages * STAGEB / kSlotBytes == 3 &&
+                              kSlotBytes + 4 * 32 * kPitch <= kStages * STAGEB),
+                  "output staging must fit the V ring");
+    stage = s_v + kSlotBytes + qg * 32 * kPitch;
+  } else {
+    stage = ((qg & 1) ? s_v : s_k) + (streams > 1 ? kSlotBytes : (qg >> 1) * 32 * kPitch);
+  }
   const float inv = st.l > 0.0f ? 1.0f / st.l : 0.0f;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -873,18 +932,27 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   }
 }
 
-// One workgroup per work list (two resident per CU): the units of list b
-// are units[bin_offset[b] .. bin_offset[b+1]), processed in order.
-template <int D>
-__global__ __launch_bounds__(kThreads, kListsPerCU) void tree_attn_kernel(SgTreeAttnArgs a) {
-  const PlanHeader* hdr = static_cast<const PlanHeader*>(a.plan_dev);
-  const AttnUnit* units = reinterpret_cast<const AttnUnit*>(hdr + 1);
-  const int32_t* bin_offset = reinterpret_cast<const int32_t*>(
-      reinterpret_cast<const MergeGroup*>(units + hdr->num_units) + hdr->num_merges);
-  const int end = bin_offset[blockIdx.x + 1];
-  for (int k = bin_offset[blockIdx.x]; k < end; ++k) {
+// One workgroup per work list: the units of list b are units[bin_offset[b] ..
+// bin_offset[b+1]), processed in order.  direct: the plan's unit records when the
+// host knows that every list is one unit (saves two round trips through the
+// plan before the first unit's), else nullptr.
+template <int D, bool kSmall>
+__global__ __launch_bounds__(Shape<kSmall>::kThreads, kSmall ? 1 : kListsPerCU) void
+tree_attn_kernel(SgTreeAttnArgs a, const AttnUnit* direct) {
+  const AttnUnit* units = direct;
+  int k = blockIdx.x;
+  int end = k + 1;
+  if (direct == nullptr) {
+    const PlanHeader* hdr = static_cast<const PlanHeader*>(a.plan_dev);
+    units = reinterpret_cast<const AttnUnit*>(hdr + 1);
+    const int32_t* bin_offset = reinterpret_cast<const int32_t*>(
+        reinterpret_cast<const MergeGroup*>(units + hdr->num_units) + hdr->num_merges);
+    k = bin_offset[blockIdx.x];
+    end = bin_offset[blockIdx.x + 1];
+  }
+  for (; k < end; ++k) {
     const AttnUnit u = units[k];
-    attn_unit<D>(a, u);
+    attn_unit<D, kSmall>(a, u);
     __syncthreads();  // LDS of this unit is free before the next one starts
   }
 }
@@ -1306,12 +1374,16 @@ extern "C" int sg_tree_attn_fwd(const SgTreeAttnArgs* args, sg_stream_t stream) 
   SG_REQUIRE(a.num_requests >= 0 && a.num_rows >= 0, "negative sizes");
   SG_REQUIRE(a.plan_units >= 0 && a.plan_merges >= 0, "negative plan sizes");
   const MergeGroup* merge_groups = nullptr;
+  const AttnUnit* direct = nullptr;
   if (a.plan_host != nullptr) {
     PlanHeader hdr;
     std::memcpy(&hdr, a.plan_host, sizeof(hdr));
     merge_groups = reinterpret_cast<const MergeGroup*>(
         static_cast<const char*>(a.plan_dev) + sizeof(PlanHeader) +
         sizeof(AttnUnit) * static_cast<size_t>(hdr.num_units));
+    if (hdr.num_units == hdr.num_bins)  // no list is empty, so every list is one unit
+      direct = reinterpret_cast<const AttnUnit*>(static_cast<const char*>(a.plan_dev) +
+                                                 sizeof(PlanHeader));
     SG_REQUIRE(hdr.magic == kPlanMagic, "plan_host is not a plan of sg_tree_attn_plan");
     SG_REQUIRE(hdr.group == G && hdr.head_dim == a.head_dim &&
                    hdr.num_kv_heads == a.num_kv_heads,
@@ -1341,24 +1413,26 @@ extern "C" int sg_tree_attn_fwd(const SgTreeAttnArgs* args, sg_stream_t stream) 
                  a.tree_row_stride >= 0 && a.tree_row_stride < (int64_t{1} << 24),
              "cache_token_stride and tree_row_stride must lie in [0, 2^24) elements");
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (a.head_dim == 128) {
-    hipLaunchKernelGGL(tree_attn_kernel<128>, dim3(a.plan_units), dim3(kThreads), 0, s, a);
-    SG_LAUNCH_CHECK();
-    if (a.plan_merges > 0) {
-      hipLaunchKernelGGL(tree_attn_merge_kernel<128>,
-                         dim3(a.plan_merges * merge_blocks_per_group(128)), dim3(kMergeThreads),
-                         0, s, a, merge_groups);
-      SG_LAUNCH_CHECK();
-    }
+  if (a.head_dim == 128 && a.plan_units <= kDefaultCUs) {
+    tree_attn_kernel<128, true><<<dim3(a.plan_units), dim3(Shape<true>::kThreads), 0, s>>>(
+        a, direct);
+  } else if (a.head_dim == 128) {
+    tree_attn_kernel<128, false><<<dim3(a.plan_units), dim3(Shape<false>::kThreads), 0, s>>>(
+        a, direct);
   } else {
-    hipLaunchKernelGGL(tree_attn_kernel<64>, dim3(a.plan_units), dim3(kThreads), 0, s, a);
-    SG_LAUNCH_CHECK();
-    if (a.plan_merges > 0) {
-      hipLaunchKernelGGL(tree_attn_merge_kernel<64>,
-                         dim3(a.plan_merges * merge_blocks_per_group(64)), dim3(kMergeThreads),
-                         0, s, a, merge_groups);
-      SG_LAUNCH_CHECK();
+    tree_attn_kernel<64, false><<<dim3(a.plan_units), dim3(Shape<false>::kThreads), 0, s>>>(
+        a, direct);
+  }
+  SG_LAUNCH_CHECK();
+  if (a.plan_merges > 0) {
+    if (a.head_dim == 128) {
+      tree_attn_merge_kernel<128><<<dim3(a.plan_merges * merge_blocks_per_group(128)),
+                                    dim3(kMergeThreads), 0, s>>>(a, merge_groups);
+    } else {
+      tree_attn_merge_kernel<64><<<dim3(a.plan_merges * merge_blocks_per_group(64)),
+                                   dim3(kMergeThreads), 0, s>>>(a, merge_groups);
     }
+    SG_LAUNCH_CHECK();
   }
   return SG_OK;
 }

@@ -169,14 +169,14 @@ def plan_attention(row_offset, prefix_len, num_q_heads: int, num_kv_heads: int,
             num_kv_heads, head_dim, target_units)
     # The plan is made once, into a buffer that holds most plans; the size it
     # reports serves a larger one.
-    host = np.zeros(_PLAN_BYTES, dtype=np.uint8)
+    host = np.empty(_PLAN_BYTES, dtype=np.uint8)
     for _ in range(2):
         rc = lib.sg_tree_attn_plan(*args, host.ctypes.data_as(ctypes.c_void_p), host.nbytes,
                                    ctypes.byref(plan_bytes), ctypes.byref(units),
                                    ctypes.byref(merges), ctypes.byref(ws))
         if rc == 0 or plan_bytes.value <= host.nbytes:
             break
-        host = np.zeros(plan_bytes.value, dtype=np.uint8)
+        host = np.empty(plan_bytes.value, dtype=np.uint8)
     _lib.check(rc, "sg_tree_attn_plan")
     host = host[:plan_bytes.value].copy()
     return AttnPlan(host, units.value, merges.value, ws.value, num_q_heads,

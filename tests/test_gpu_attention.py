@@ -147,6 +147,24 @@ def test_runs_of_consecutive_nodes_and_unseen_tree_tiles(device, oracle, nodes, 
     _assert_close(got, oracle.attention_dense(q, ks, vs, kt, vt, wl.parents))
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9, 17, 32, 40])
+def test_small_waves_at_the_ring_edges(device, oracle, rows):
+    # Fewer units than CUs at D 128: prefixes of every number of tiles around
+    # the ring of eight, one to four q-groups and a second row tile.
+    tree = [-1] + [(k * 5) % k if k > 1 else 0 for k in range(1, rows)]
+    lengths = np.asarray([0, 1, 31, 32, 33, 64, 65, 96, 128, 160, 191, 192, 224, 225, 255, 256,
+                          257, 288, 320, 352, 383, 416, 449, 512], np.int32)
+    n = len(lengths)
+    wl = W.AttentionWorkload("ring", 8, 2, 128, lengths, [tree] * n, [[0] * (rows - 1)] * n, 576)
+    tensors, dev, meta = _inputs(wl, device, rows)
+    for units in (0, 16):  # a unit per list, and lists of several units
+        got, plan = _run(wl, dev, meta, device, units)
+        assert plan.units <= 256
+        ks, vs = _prefix_lists(wl, tensors)
+        q, kc, vc, kt, vt = tensors
+        _assert_close(got, oracle.attention_dense(q, ks, vs, kt, vt, wl.parents))
+
+
 def test_strided_query_and_output_views(device, oracle):
     wl = W.tiny_attention_workload(seed=3, num_q_heads=8, num_kv_heads=2, head_dim=128)
     tensors, dev, meta = _inputs(wl, device, 14)
