@@ -27,13 +27,13 @@
 // own order, and 1/sqrt and sincos are the device's, so a normed or rotated
 // value can still differ from transformers' by one bf16 ulp.
 //
-// All of them are bound by HBM once each load of a thread is issued before the
-// first is used and the conversions to bf16 are gfx950's own.  One layer's four
-// calls over 2,048 rows (hidden 4096, intermediate 12288, 32 q / 8 kv heads of
-// 128; 336 MB): 81.4 -> 77.4 us, and 72.8 us (4.6 TB/s, a large copy reaches 4.9)
-// with non-temporal loads.  Non-temporal stores were 3.5 us faster still here
-// and 25 us slower in a 512-row decoder of four layers, whose next kernel reads
-// the stored rows from the caches: not used.
+// All of them are bound by HBM (or the last-level cache, where the inputs are
+// still there) once each load of a thread is issued before the first is used and
+// the conversions to bf16 are gfx950's own.  One layer's four calls (hidden 4096,
+// intermediate 12288, 32 q / 8 kv heads of 128): 2,048 rows (336 MB) 79 -> 65.6
+// us (80.3 -> 77.0 on inputs that no cache holds), 4,096 rows 140 -> 133, 1,024 rows 39.5 -> 38.4.  Non-temporal stores: 3.5
+// us less over 2,048 rows, 25 us more in a 512-row decoder of four layers, where
+// the next kernel reads the stored rows from the caches: not used.
 #include <algorithm>
 #include <cmath>
 
@@ -44,10 +44,11 @@ namespace {
 
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
-// 16 bytes that this kernel alone reads: the non-temporal hint keeps them from
-// displacing the outputs, which the next kernel reads, in the caches.
-__device__ __forceinline__ uint4 ntload(const void* p) {
-  const u32x4 v = __builtin_nontemporal_load(static_cast<const u32x4*>(p));
+// 16 bytes, with the non-temporal hint when kStream.
+template <bool kStream>
+__device__ __forceinline__ uint4 load16(const void* p) {
+  const u32x4* q = static_cast<const u32x4*>(p);
+  const u32x4 v = kStream ? __builtin_nontemporal_load(q) : *q;
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
@@ -95,9 +96,9 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
   for (int c = 0; c < kChunks; ++c) {
     const int e = 8 * (threadIdx.x + c * kNormThreads);
     const bool live = e < hidden;
-    s[c] = live ? ntload(xr + e) : make_uint4(0u, 0u, 0u, 0u);
+    s[c] = live ? *reinterpret_cast<const uint4*>(xr + e) : make_uint4(0u, 0u, 0u, 0u);
     if (kResidual)
-      b[c] = live ? ntload(rr + e) : make_uint4(0u, 0u, 0u, 0u);
+      b[c] = live ? *reinterpret_cast<const uint4*>(rr + e) : make_uint4(0u, 0u, 0u, 0u);
   }
 #pragma unroll
   for (int c = 0; c < kChunks; ++c) {
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(kNormThreads) void qk_norm_rope_kernel(
 #pragma unroll
     for (int b = 0; b < kBatch; ++b) {
       const int h = h0 + b * waves * HPW + slot;
-      raw[b] = h < heads ? ntload(src + static_cast<int64_t>(h) * D)
+      raw[b] = h < heads ? *reinterpret_cast<const uint4*>(src + static_cast<int64_t>(h) * D)
                          : make_uint4(0u, 0u, 0u, 0u);
     }
   };
@@ -266,10 +267,18 @@ __global__ __launch_bounds__(kNormThreads) void qk_norm_rope_kernel(
 }
 
 // out[r, i] = bf16(bf16(silu(gate[r, i])) * up[r, i]); gate = gu[r, :I],
-// up = gu[r, I:2I].  A workgroup takes kSiluChunks * 256 chunks of 8 elements
-// of one row (parts = workgroups per row), so that the row is one scalar
-// division and a thread has four loads in flight.
-constexpr int kSiluChunks = 2;
+// up = gu[r, I:2I].  A workgroup takes 256 chunks of 8 elements of one row (parts =
+// workgroups per row), so that finding the row is one scalar division; two
+// chunks a thread measured 4 % slower.
+// kStream: non-temporal loads, for calls that move kStreamBytes or more.  Below,
+// what the projection before has just written is still in the 256 MB last-level
+// cache and the hint costs time; above, most of it is not, and the hint keeps
+// what is left for the next kernel.  The four stages of one layer (hidden 4096,
+// intermediate 12288) without / with the hint: 768 rows 32.3 / 35.6 us, 1,536
+// rows 51 / 58, 2,048 rows (151 MB here) 77 / 65.6, 4,096 rows 135 / 133.
+constexpr int64_t kStreamBytes = int64_t{128} << 20;
+constexpr int kSiluPart = 8 * 256;  // elements of a workgroup's part of a row
+template <bool kStream>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gu,
                                                        int64_t gu_stride, int inter,
                                                        uint16_t* __restrict__ out,
@@ -278,31 +287,21 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
   for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
     const int64_t row = item / parts;
     const uint32_t part = static_cast<uint32_t>(item - row * parts);
-    const uint32_t e0 = 8 * (part * kSiluChunks * 256 + threadIdx.x);
-    const uint16_t* gr = gu + row * gu_stride;
-    uint4 g[kSiluChunks], u[kSiluChunks];
+    const uint32_t e = part * kSiluPart + 8 * threadIdx.x;
+    if (e >= static_cast<uint32_t>(inter)) continue;
+    const uint16_t* gr = gu + row * gu_stride + e;
+    const uint4 g = load16<kStream>(gr);
+    const uint4 u = load16<kStream>(gr + inter);
+    const uint32_t gv[4] = {g.x, g.y, g.z, g.w};
+    const uint32_t uv[4] = {u.x, u.y, u.z, u.w};
+    uint32_t o[4];
 #pragma unroll
-    for (int c = 0; c < kSiluChunks; ++c) {
-      const uint32_t e = e0 + c * 8 * 256;
-      const bool live = e < static_cast<uint32_t>(inter);
-      g[c] = live ? ntload(gr + e) : make_uint4(0u, 0u, 0u, 0u);
-      u[c] = live ? ntload(gr + inter + e) : make_uint4(0u, 0u, 0u, 0u);
+    for (int q = 0; q < 4; ++q) {
+      const Pair x = unpack(gv[q]), up = unpack(uv[q]);
+      const Pair s = bf16r(x.lo / (1.0f + expf(-x.lo)), x.hi / (1.0f + expf(-x.hi)));
+      o[q] = pack_bf16x2(s.lo * up.lo, s.hi * up.hi);
     }
-#pragma unroll
-    for (int c = 0; c < kSiluChunks; ++c) {
-      const uint32_t e = e0 + c * 8 * 256;
-      if (e >= static_cast<uint32_t>(inter)) continue;
-      const uint32_t gv[4] = {g[c].x, g[c].y, g[c].z, g[c].w};
-      const uint32_t uv[4] = {u[c].x, u[c].y, u[c].z, u[c].w};
-      uint32_t o[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const Pair x = unpack(gv[q]), up = unpack(uv[q]);
-        const Pair s = bf16r(x.lo / (1.0f + expf(-x.lo)), x.hi / (1.0f + expf(-x.hi)));
-        o[q] = pack_bf16x2(s.lo * up.lo, s.hi * up.hi);
-      }
-      *reinterpret_cast<uint4*>(out + row * out_stride + e) = make_uint4(o[0], o[1], o[2], o[3]);
-    }
+    *reinterpret_cast<uint4*>(out + row * out_stride + e) = make_uint4(o[0], o[1], o[2], o[3]);
   }
 }
 
@@ -426,13 +425,16 @@ extern "C" int sg_silu_mul(const void* gate_up_dev, int64_t gate_up_row_stride,
                  out_row_stride >= intermediate && (gate_up_row_stride | out_row_stride) % 8 == 0,
              "row strides must cover the rows and be multiples of 8");
   SG_REQUIRE(aligned16(gate_up_dev) && aligned16(out_dev), "tensors must be 16-byte aligned");
-  constexpr int kPart = 8 * 256 * kSiluChunks;  // elements of a workgroup's part of a row
-  const uint32_t parts = (static_cast<uint32_t>(intermediate) + kPart - 1) / kPart;
+  const uint32_t parts = (static_cast<uint32_t>(intermediate) + kSiluPart - 1) / kSiluPart;
   const int64_t items = static_cast<int64_t>(num_rows) * parts;
-  silu_mul_kernel<<<dim3(static_cast<unsigned>(std::min<int64_t>(items, 1 << 20))), dim3(256), 0,
-                    static_cast<hipStream_t>(stream)>>>(
-      static_cast<const uint16_t*>(gate_up_dev), gate_up_row_stride, intermediate,
-      static_cast<uint16_t*>(out_dev), out_row_stride, parts, items);
+  auto go = [&](auto kernel) {
+    kernel<<<dim3(static_cast<unsigned>(std::min<int64_t>(items, 1 << 20))), dim3(256), 0,
+             static_cast<hipStream_t>(stream)>>>(
+        static_cast<const uint16_t*>(gate_up_dev), gate_up_row_stride, intermediate,
+        static_cast<uint16_t*>(out_dev), out_row_stride, parts, items);
+  };
+  const int64_t bytes = static_cast<int64_t>(num_rows) * intermediate * 6;  // two in, one out
+  bytes >= kStreamBytes ? go(silu_mul_kernel<true>) : go(silu_mul_kernel<false>);
   SG_LAUNCH_CHECK();
   return SG_OK;
 }
