@@ -8,7 +8,8 @@
 // reference's dense packed mask (continuous_tree_block_decode.py:500-546 and
 // tree.py:19-26) evaluated without materialising the mask or copying prefixes.
 //
-// Decomposition (MI355X, two 4-wave workgroups per CU):
+// Decomposition (MI355X, two 4-wave workgroups per CU, or one of eight waves where
+// a launch has no more workgroups than CUs; `Shape`):
 //   unit      = (request, kv head, tile of up to 128/G query rows = 128 query
 //               vectors = four 32-vector q-groups, range of prefix keys); the
 //               unit that ends a request's key range also covers its tree rows;
@@ -17,10 +18,11 @@
 //               end of the launch;
 //   window    = one barrier; consumes two 32-key K and V tiles, moved
 //               HBM -> LDS by global_load_lds_dwordx4 (no register staging)
-//               into 4-tile rings issued one window ahead;
+//               into 4-tile rings issued one window ahead (eight-wave form:
+//               8-tile rings, three windows);
 //   wave      = one q-group over both tiles of every window (3-4 q-groups)
 //               or one of two key streams of a q-group taking one tile of
-//               each window (1-2 q-groups).  Every wave runs its own online
+//               each window (1-2 q-groups; with eight waves, always).  Every wave runs its own online
 //               softmax; the key streams of a q-group are merged through LDS
 //               at the end of the unit.
 // Per 32-key block a wave computes S^T = K Q^T with v_mfma_f32_32x32x16_bf16
