@@ -8,8 +8,8 @@
 // reference's dense packed mask (continuous_tree_block_decode.py:500-546 and
 // tree.py:19-26) evaluated without materialising the mask or copying prefixes.
 //
-// Decomposition (MI355X, two 4-wave workgroups per CU, or one of eight waves where
-// a launch has no more workgroups than CUs; `Shape`):
+// Decomposition (MI355X, two 4-wave workgroups per CU, or one of eight waves for
+// launches of few small units; `Shape`):
 //   unit      = (request, kv head, tile of up to 128/G query rows = 128 query
 //               vectors = four 32-vector q-groups, range of prefix keys); the
 //               unit that ends a request's key range also covers its tree rows;
@@ -22,7 +22,7 @@
 //               8-tile rings, three windows);
 //   wave      = one q-group over both tiles of every window (3-4 q-groups)
 //               or one of two key streams of a q-group taking one tile of
-//               each window (1-2 q-groups; with eight waves, always).  Every wave runs its own online
+//               each window (1-2 q-groups).  Every wave runs its own online
 //               softmax; the key streams of a q-group are merged through LDS
 //               at the end of the unit.
 // Per 32-key block a wave computes S^T = K Q^T with v_mfma_f32_32x32x16_bf16
@@ -56,12 +56,18 @@ typedef __attribute__((address_space(3))) short4_t lds_short4;
 constexpr int kQPerUnit = 128;
 constexpr int kTileKeys = 32;                   // keys per tile: one 32-key MFMA block
 constexpr int kListsPerCU = 2;                  // resident workgroups per CU
-// Shape of a workgroup.  kSmall: launches of at most one workgroup per CU at
-// D = 128, where a workgroup has all of its CU: eight waves (two key streams for
-// four q-groups, so two waves per matrix unit) and copies three windows ahead
-// (137 KB of LDS).  16 requests, 512 rows, 354-2,036 cached tokens, 32 q / 8 kv
-// heads: 38.3 -> 36.5 us (37.1 us one window ahead; 43.4 us with four waves).
-// D = 64 measured equal and keeps four waves.
+// Shape of a workgroup.  kSmall: launches at D = 128 of at most one workgroup
+// per CU, whose units all have at most two q-groups.  Such a workgroup has all
+// of its CU and waits mostly for its copies: eight waves issue them, three
+// windows ahead (137 KB of LDS).  32 q / 8 kv heads, four-wave / eight-wave form:
+// 31 one-row requests at 500-4,000 cached tokens 83.8 / 64.3 us, 16 of 16 rows
+// at 2,000-8,000 79.5 / 71.8 us; 16 kv heads of one query head, 12 requests of
+// 16-32 rows 57.9 / 48.6 us.  The rule stops at two q-groups because both forms
+// then give every q-group the same two key streams, so a row's result is the
+// same bits in either; eight waves over 3-4 q-groups (36.1 instead of 37.6 us for
+// 16 requests of 16-64 rows) round the probabilities against the maxima
+// of other streams.  D = 64 measured equal and keeps four waves.
+constexpr int kSmallVectors = 64;  // query vectors of a unit of two q-groups
 template <bool kSmall>
 struct Shape {
   static constexpr int kWaves = kSmall ? 8 : 4;
@@ -92,7 +98,7 @@ struct PlanHeader {
   int32_t num_requests;   // n and R = row_offset[n] of the wave the plan was built for
   int32_t num_rows;
   int32_t num_kv_heads;
-  int32_t reserved0;
+  int32_t unit_rows;      // most rows of a unit; 0: not known (plans made before the field)
   uint64_t meta_hash;     // FNV-1a over row_offset[0..n] and prefix_len[0..n-1]
   int32_t reserved[2];
 };
@@ -182,7 +188,7 @@ __host__ __device__ constexpr int swz_v(int r) {
 // the row tiles of a larger tree re-read the same K/V and keep it cached.  Issued as inline assembly so that the compiler does not
 // model it: its automatic waits would otherwise stall the first LDS read of the
 // other pipeline stage on this in-flight copy.  The kernel waits for the DMAs
-// explicitly (s_waitcnt vmcnt(0)) before the barrier that publishes the tile.
+// explicitly (s_waitcnt vmcnt) before the barrier that publishes the tile.
 // m0 (the LDS base of the copy) is written here and declared clobbered.
 template <bool kStream>
 __device__ __forceinline__ void dma16(const void* gbase, uint32_t voff, uint32_t lds) {
@@ -327,11 +333,12 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   const int col = lane & 31;
   const int nq = (u.row_count * G + 31) / 32;   // q-groups in use, 1..4
   // Every window (one barrier) consumes two consecutive 32-key tiles.  With
-  // 1-2 q-groups (1-4 in eight waves) two waves share a q-group ("key streams") and take one tile
+  // 1-2 q-groups two waves share a q-group ("key streams") and take one tile
   // each; their results are merged at the end of the unit.  With 3-4 q-groups
-  // every wave takes both tiles, one after the other.  Waves beyond
-  // nq*streams repeat stream 0's work on the same LDS data and discard it (in
-  // the small form they only copy).
+  // every wave takes both tiles, one after the other (in the small form, which
+  // meets them only if the device's plan is not the host's, two streams).  Waves
+  // beyond nq*streams repeat stream 0's work on the same LDS data and discard it
+  // (in the small form they only copy).
   const int streams = 2 * nq <= kWaves ? 2 : 1;
   const bool both = !kSmall && streams == 1;
   const int qg = wave % nq;
@@ -712,8 +719,9 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
   };
 
   // Steady state: windows whose current tiles and the tiles of their QK
-  // products are full prefix tiles need no mask, and the ring stages are
-  // compile-time constants in loops unrolled by two windows (the ring size).
+  // products are full prefix tiles need no mask, and the ring stages of the
+  // four-wave form are compile-time constants in loops unrolled by two windows
+  // (the ring size).
   // The last tile a window's QK products read is 2i+koff-1.
   const int steady_end = max(0, (tiles_full - koff + 2) / 2);
   int i = 0;
@@ -802,7 +810,7 @@ __device__ __forceinline__ void attn_unit(const SgTreeAttnArgs& a, const AttnUni
 
 
   // Merge the key streams of each q-group through LDS (the ring is free now).
-  // Slot k (k = (ks-1)*nq + qg < 6) lives at float offset k*STATE*64 of s_k|s_v.
+  // Slot k (k = (ks-1)*nq + qg < kWaves/2) lives at float offset k*STATE*64 of s_k|s_v.
   auto merge_slot = [&](int k) -> float* {
     constexpr int kPerBuf = (kStages * STAGEB) / (STATE * 64 * 4);
     unsigned char* buf = (k < kPerBuf) ? s_k : s_v;
@@ -1328,6 +1336,7 @@ extern "C" int sg_tree_attn_plan(int32_t num_requests, const int32_t* row_offset
   hdr.num_requests = num_requests;
   hdr.num_rows = num_requests > 0 ? row_offset_host[num_requests] : 0;
   hdr.num_kv_heads = num_kv_heads;
+  for (const AttnUnit& u : units) hdr.unit_rows = std::max(hdr.unit_rows, u.row_count);
   hdr.meta_hash = meta_hash(num_requests, row_offset_host, prefix_len_host);
   char* out = static_cast<char*>(plan_host);
   std::memcpy(out, &hdr, sizeof(hdr));
@@ -1377,6 +1386,7 @@ extern "C" int sg_tree_attn_fwd(const SgTreeAttnArgs* args, sg_stream_t stream) 
   SG_REQUIRE(a.plan_units >= 0 && a.plan_merges >= 0, "negative plan sizes");
   const MergeGroup* merge_groups = nullptr;
   const AttnUnit* direct = nullptr;
+  bool small_units = false;
   if (a.plan_host != nullptr) {
     PlanHeader hdr;
     std::memcpy(&hdr, a.plan_host, sizeof(hdr));
@@ -1386,6 +1396,7 @@ extern "C" int sg_tree_attn_fwd(const SgTreeAttnArgs* args, sg_stream_t stream) 
     if (hdr.num_units == hdr.num_bins)  // no list is empty, so every list is one unit
       direct = reinterpret_cast<const AttnUnit*>(static_cast<const char*>(a.plan_dev) +
                                                  sizeof(PlanHeader));
+    small_units = hdr.unit_rows >= 1 && hdr.unit_rows <= kSmallVectors / G;
     SG_REQUIRE(hdr.magic == kPlanMagic, "plan_host is not a plan of sg_tree_attn_plan");
     SG_REQUIRE(hdr.group == G && hdr.head_dim == a.head_dim &&
                    hdr.num_kv_heads == a.num_kv_heads,
@@ -1415,7 +1426,7 @@ extern "C" int sg_tree_attn_fwd(const SgTreeAttnArgs* args, sg_stream_t stream) 
                  a.tree_row_stride >= 0 && a.tree_row_stride < (int64_t{1} << 24),
              "cache_token_stride and tree_row_stride must lie in [0, 2^24) elements");
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (a.head_dim == 128 && a.plan_units <= kDefaultCUs) {
+  if (a.head_dim == 128 && small_units && a.plan_units <= kDefaultCUs) {
     tree_attn_kernel<128, true><<<dim3(a.plan_units), dim3(Shape<true>::kThreads), 0, s>>>(
         a, direct);
   } else if (a.head_dim == 128) {

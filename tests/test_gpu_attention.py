@@ -165,6 +165,44 @@ def test_small_waves_at_the_ring_edges(device, oracle, rows):
         _assert_close(got, oracle.attention_dense(q, ks, vs, kt, vt, wl.parents))
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
+def test_workgroup_forms_agree_bit_for_bit(device, rows):
+    """Units of at most 64 query vectors: a launch of few workgroups (eight
+    waves each where the host's plan tells the units' sizes) gives a row the
+    bits of the four-wave form, at prefixes around both rings, split or not."""
+    tree = [-1] + [(k * 5) % k if k > 1 else 0 for k in range(1, rows)]
+    lengths = np.asarray([0, 1, 31, 32, 64, 65, 127, 129, 191, 192, 224, 225, 255, 256, 257, 320,
+                          383, 449, 512, 1000, 1027, 3000], np.int32)
+    n = len(lengths)
+    wl = W.AttentionWorkload("forms", 8, 2, 128, lengths, [tree] * n, [[0] * (rows - 1)] * n, 3072)
+    _, (q, kc, vc, kt, vt), meta = _inputs(wl, device, rows)
+    for units in (0, 16):
+        plan = ops.plan_attention(wl.row_offset, wl.prefix_len, 8, 2, 128, units).to(device)
+        assert plan.units <= 256 and (units or plan.merges)
+        call = ops.prepare_tree_attention(q, kc, vc, kt, vt, meta["row_offset"],
+                                          meta["prefix_start"], meta["prefix_len"],
+                                          meta["parent"], plan)
+        eight = call().clone()
+        four = call.set(plan_host=None)()
+        torch.cuda.synchronize()
+        assert torch.equal(eight, four)
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 32])
+def test_rows_do_not_depend_on_the_number_of_lists(device, rows):
+    """The same 320 units as 320 work lists and packed onto 200: a row's result
+    is the same bits, whatever the launch's workgroup count selects."""
+    tree = [-1] + [(k * 5) % k if k > 1 else 0 for k in range(1, rows)]
+    n = 40
+    lengths = np.asarray([(37 * i) % 128 for i in range(n)], np.int32)  # too short to split
+    wl = W.AttentionWorkload("lists", 32, 8, 128, lengths, [tree] * n, [[0] * (rows - 1)] * n, 160)
+    _, dev, meta = _inputs(wl, device, rows)
+    own, plan = _run(wl, dev, meta, device)
+    packed, hinted = _run(wl, dev, meta, device, 200)
+    assert plan.units == 320 and hinted.units <= 200 and plan.merges == hinted.merges == 0
+    assert torch.equal(own, packed)
+
+
 def test_strided_query_and_output_views(device, oracle):
     wl = W.tiny_attention_workload(seed=3, num_q_heads=8, num_kv_heads=2, head_dim=128)
     tensors, dev, meta = _inputs(wl, device, 14)
