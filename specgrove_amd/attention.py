@@ -50,7 +50,6 @@ class PackedTreeMask:
     row_offset_host: np.ndarray
     prefix_len_host: np.ndarray
     plans: dict = field(default_factory=dict)
-    streams: set = field(default_factory=set)  # handles of the streams that ordered the copies
 
     @property
     def num_rows(self) -> int:
@@ -61,30 +60,12 @@ class PackedTreeMask:
         shared by every layer)."""
         key = (num_q_heads, num_kv_heads, head_dim)
         if key not in self.plans:
-            self.plans[key] = ops.plan_attention(
-                self.row_offset_host, self.prefix_len_host, num_q_heads, num_kv_heads,
-                head_dim).to(self.row_offset.device, non_blocking=True)
-            self._ordered_here()
-        self._join()
+            plan = ops.plan_attention(self.row_offset_host, self.prefix_len_host, num_q_heads,
+                                      num_kv_heads, head_dim)
+            plan.device = ops.upload(plan.host, self.row_offset.device)
+            plan.workspace = plan.new_workspace()
+            self.plans[key] = plan
         return self.plans[key]
-
-    def _ordered_here(self) -> None:
-        """The current stream ordered a copy of this mask."""
-        if self.row_offset.is_cuda:
-            self.streams.add(ops._stream_handle())
-
-    def _join(self) -> None:
-        """The mask's copies are ordered by the streams that were current when
-        it and its plans were made; any other stream waits for those first."""
-        if not self.streams:
-            return
-        here = ops._stream_handle()
-        for handle in self.streams:
-            if handle != here:
-                device = self.row_offset.device
-                torch.cuda.current_stream(device).wait_stream(
-                    torch.cuda.ExternalStream(handle, device=device) if handle
-                    else torch.cuda.default_stream(device))
 
 
 def _parents_precede(flat: np.ndarray, row_offset: np.ndarray, parents_list) -> bool:
@@ -132,7 +113,7 @@ def build_tree_mask(pool, caches: Sequence, parents_list: Sequence[Sequence[int]
     host = np.concatenate([prefix_start.astype(np.int64), words32.view(np.int64)])
     meta = ops.upload(host, dev)
     meta32 = meta[n:].view(torch.int32)
-    mask = PackedTreeMask(
+    return PackedTreeMask(
         pool=pool,
         row_offset=meta32[:n + 1],
         parent=meta32[2 * n + 1:2 * n + 1 + parent.size],
@@ -141,8 +122,6 @@ def build_tree_mask(pool, caches: Sequence, parents_list: Sequence[Sequence[int]
         row_offset_host=row_offset,
         prefix_len_host=prefix_len,
     )
-    mask._ordered_here()
-    return mask
 
 
 def pack_block_inputs(states, blocks, cache_lengths: Sequence[int],

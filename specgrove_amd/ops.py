@@ -63,14 +63,28 @@ class PreparedCall:
         return self
 
 
+_upload_streams: dict = {}  # device index -> the stream of upload()'s copies
+
+
 def upload(array: np.ndarray, device) -> torch.Tensor:
-    """A host array on the device, copied in stream order from pinned memory:
-    the host does not wait for the stream's earlier work.  (While a stream is
-    captured the copy is a plain one, which capture refuses.)"""
+    """A host array on the device, complete on return: any stream, graph
+    capture or thread may read it without waiting.  The copy runs on a stream
+    of its own into memory of that stream, so the host waits for the copy (36
+    to 39 us for 32 KiB; 24 us on the current stream while it is idle) and not
+    for the current stream's earlier work.  (While a stream is captured the
+    copy is a plain one, which capture refuses.)"""
     host = torch.from_numpy(array)
-    if torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+    device = torch.device(device)
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
         return host.to(device)
-    return host.pin_memory().to(device, non_blocking=True)
+    index = torch.cuda.current_device() if device.index is None else device.index
+    stream = _upload_streams.get(index)
+    if stream is None:
+        stream = _upload_streams.setdefault(index, torch.cuda.Stream(index))
+    with torch.cuda.stream(stream):
+        copy = host.to(device)
+    copy.record_stream(torch.cuda.current_stream(index))
+    return copy
 
 
 def _require(cond: bool, message: str) -> None:
@@ -138,16 +152,18 @@ class AttnPlan:
     def num_rows(self) -> int:
         return int(self.header[9])
 
-    def to(self, device, non_blocking: bool = False) -> "AttnPlan":
-        """Copy the plan to the device and allocate its workspace (the fp32
-        partial results of split units; every slot is written before the merge
-        kernel reads it, so its initial contents do not matter).  With
-        ``non_blocking`` the copy is only ordered on the current stream."""
-        self.device = upload(self.host, device) if non_blocking else \
-            torch.from_numpy(self.host).to(device, non_blocking=False)
-        self.workspace = torch.zeros(max(self.workspace_bytes, 16), dtype=torch.uint8,
-                                     device=device)
+    def to(self, device) -> "AttnPlan":
+        """Copy the plan to the device and allocate its workspace."""
+        self.device = torch.from_numpy(self.host).to(device, non_blocking=False)
+        self.workspace = self.new_workspace()
         return self
+
+    def new_workspace(self) -> torch.Tensor:
+        """Device memory of one call at a time: the fp32 partial results of
+        split units (every slot is written before the merge kernel reads it,
+        so its initial contents do not matter)."""
+        return torch.zeros(max(self.workspace_bytes, 16), dtype=torch.uint8,
+                           device=self.device.device)
 
 
 _PLAN_BYTES = 1 << 16  # about 1,300 units

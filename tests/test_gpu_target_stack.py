@@ -343,6 +343,59 @@ def test_a_mask_used_on_another_stream_waits_for_its_copies(device, planned_here
     torch.cuda.synchronize()
 
 
+def _mask_case(device, dim=64, seed=1):
+    from types import SimpleNamespace
+    lengths, tree = [300, 517, 64], [-1, 0, 1, 1, 0]
+    g = torch.Generator(device).manual_seed(seed)
+    pool = SimpleNamespace(lengths=lengths, capacity=576)
+    pool.key_storage = [torch.randn((2, 3 * 576, dim), generator=g, device=device)
+                        .to(torch.bfloat16)]
+    pool.value_storage = [torch.randn_like(pool.key_storage[0])]
+    caches = [SimpleNamespace(slot=i) for i in range(3)]
+    q, k, v = (torch.randn((1, h, 15, dim), generator=g, device=device).to(torch.bfloat16)
+               for h in (4, 2, 2))
+    return pool, caches, [tree] * 3, (SimpleNamespace(layer_idx=0), q, k, v)
+
+
+def test_a_mask_and_its_plan_are_complete_on_return(device):
+    """Their fields are read on another stream, at once: copies left on the
+    stream that was current when they were made would come after its work."""
+    from specgrove_amd import attention
+    pool, caches, trees, _ = _mask_case(device)
+    side = torch.cuda.Stream()
+    busy = torch.randn((4096, 4096), device=device)
+    attention.build_tree_mask(pool, caches, trees, device).plan(4, 2, 64)
+    torch.cuda.synchronize()
+    for _ in range(40):
+        busy = busy @ busy * 1e-3
+    mask = attention.build_tree_mask(pool, caches, trees, device)
+    plan = mask.plan(4, 2, 64)
+    with torch.cuda.stream(side):
+        got = [t.clone() for t in (mask.row_offset, mask.prefix_start, mask.prefix_len,
+                                   mask.parent, plan.device)]
+    side.synchronize()
+    want = [[0, 5, 10, 15], [0, 576, 1152], pool.lengths, sum(trees, []), plan.host.tolist()]
+    torch.cuda.synchronize()
+    assert [t.tolist() for t in got] == want
+
+
+def test_a_mask_made_ahead_is_used_in_a_capture(device):
+    from specgrove_amd import attention
+    pool, caches, trees, args = _mask_case(device, dim=128)
+    mask = attention.build_tree_mask(pool, caches, trees, device)
+    want = attention.tree_attention_forward(*args, mask)[0].clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):  # captures on a stream of its own
+        out = attention.tree_attention_forward(*args, mask)[0]
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        attention.tree_attention_forward(*args, mask)
+
+
 def test_decode_loop_runs_on_the_stack(device):
     transformers = pytest.importorskip("transformers")
     from specgrove_amd import decode, scheduler
