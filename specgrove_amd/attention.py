@@ -56,16 +56,22 @@ class PackedTreeMask:
         return int(self.row_offset_host[-1])
 
     def plan(self, num_q_heads: int, num_kv_heads: int, head_dim: int) -> ops.AttnPlan:
-        """Work plan of this wave for a head configuration (built once and
-        shared by every layer)."""
+        """Work plan of this wave for a head configuration.  It is built and
+        copied once; each call returns it with a workspace of its own, and
+        lets the wave's tensors outlive the current stream's use of them."""
         key = (num_q_heads, num_kv_heads, head_dim)
         if key not in self.plans:
             plan = ops.plan_attention(self.row_offset_host, self.prefix_len_host, num_q_heads,
                                       num_kv_heads, head_dim)
             plan.device = ops.upload(plan.host, self.row_offset.device)
-            plan.workspace = plan.new_workspace()
             self.plans[key] = plan
-        return self.plans[key]
+        plan = self.plans[key]
+        if plan.device.is_cuda:
+            stream = torch.cuda.current_stream(plan.device.device)
+            for t in (plan.device, self.row_offset, self.parent, self.prefix_start,
+                      self.prefix_len):
+                t.record_stream(stream)
+        return plan.with_workspace()
 
 
 def _parents_precede(flat: np.ndarray, row_offset: np.ndarray, parents_list) -> bool:

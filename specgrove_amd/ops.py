@@ -9,7 +9,7 @@ raise ValueError before anything is launched; launch errors raise RuntimeError.
 from __future__ import annotations
 
 import ctypes
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import numpy as np
 import torch
@@ -153,17 +153,20 @@ class AttnPlan:
         return int(self.header[9])
 
     def to(self, device) -> "AttnPlan":
-        """Copy the plan to the device and allocate its workspace."""
+        """Copy the plan to the device and allocate its workspace (the fp32
+        partial results of split units; every slot is written before the merge
+        kernel reads it, so its initial contents do not matter)."""
         self.device = torch.from_numpy(self.host).to(device, non_blocking=False)
-        self.workspace = self.new_workspace()
+        self.workspace = torch.zeros(max(self.workspace_bytes, 16), dtype=torch.uint8,
+                                     device=device)
         return self
 
-    def new_workspace(self) -> torch.Tensor:
-        """Device memory of one call at a time: the fp32 partial results of
-        split units (every slot is written before the merge kernel reads it,
-        so its initial contents do not matter)."""
-        return torch.zeros(max(self.workspace_bytes, 16), dtype=torch.uint8,
-                           device=self.device.device)
+    def with_workspace(self) -> "AttnPlan":
+        """The same plan on the device with a workspace of its own, of the
+        current stream's memory: calls that can overlap, as on two streams,
+        must not share one."""
+        return replace(self, workspace=torch.empty(
+            max(self.workspace_bytes, 16), dtype=torch.uint8, device=self.device.device))
 
 
 _PLAN_BYTES = 1 << 16  # about 1,300 units

@@ -379,6 +379,28 @@ def test_a_mask_and_its_plan_are_complete_on_return(device):
     assert [t.tolist() for t in got] == want
 
 
+def test_one_mask_on_two_streams_at_once(device):
+    from specgrove_amd import attention
+    cases = [_mask_case(device, dim=128, seed=s) for s in (1, 2)]
+    pool, caches, trees, _ = cases[0]
+    mask = attention.build_tree_mask(pool, caches, trees, device)
+    args = [case[3] for case in cases]
+    want = [attention.tree_attention_forward(*a, mask)[0].clone() for a in args]
+    assert mask.plan(4, 2, 128).merges > 0
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream() for _ in args], [[], []]
+    for _ in range(8):
+        for k, a in enumerate(args):
+            with torch.cuda.stream(streams[k]):
+                got[k].append(attention.tree_attention_forward(*a, mask)[0])
+    del mask  # its memory must not be reused before both streams are done
+    junk = [attention.build_tree_mask(pool, caches, trees, device) for _ in range(4)]
+    torch.cuda.synchronize()
+    for k in range(2):
+        assert all(torch.equal(t, want[k]) for t in got[k])
+    del junk
+
+
 def test_a_mask_made_ahead_is_used_in_a_capture(device):
     from specgrove_amd import attention
     pool, caches, trees, args = _mask_case(device, dim=128)

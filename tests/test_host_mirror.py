@@ -92,6 +92,18 @@ def test_packed_inputs_match_the_reference_dense_mask(oracle):
     assert m.prefix_start.tolist() == [i * pool.capacity for i in range(4)]
 
 
+def test_plans_of_one_mask_share_their_records_and_no_workspace():
+    # Two streams of one wave may run at once; split units write partials.
+    pool = SimpleNamespace(lengths=[2000, 700], capacity=2048)
+    mask = attention.build_tree_mask(pool, [SimpleNamespace(slot=i) for i in range(2)],
+                                     [[-1, 0, 0], [-1]], "cpu")
+    a, b = mask.plan(32, 8, 128), mask.plan(32, 8, 128)
+    assert a.merges > 0 and a.workspace.numel() >= a.workspace_bytes > 16
+    assert a.host is b.host and a.device is b.device
+    assert a.workspace.data_ptr() != b.workspace.data_ptr()
+    assert b.workspace.numel() == a.workspace.numel()
+
+
 def test_packed_inputs_reject_bad_trees_and_foreign_pools():
     rng = np.random.default_rng(1)
     pool, _ = _pool([5, 6])
