@@ -30,10 +30,12 @@
 // All of them are bound by HBM (or the last-level cache, where the inputs are
 // still there) once each load of a thread is issued before the first is used and
 // the conversions to bf16 are gfx950's own.  One layer's four calls (hidden 4096,
-// intermediate 12288, 32 q / 8 kv heads of 128): 2,048 rows (336 MB) 79 -> 65.6
-// us (80.3 -> 77.0 on inputs that no cache holds), 4,096 rows 140 -> 133, 1,024 rows 39.5 -> 38.4.  Non-temporal stores: 3.5
-// us less over 2,048 rows, 25 us more in a 512-row decoder of four layers, where
-// the next kernel reads the stored rows from the caches: not used.
+// intermediate 12288, 32 q / 8 kv heads of 128) over 2,048 rows (336 MB), on new
+// inputs in each call: 80.3 -> 75.4 us (the fused stages by themselves, repeated
+// over one set of tensors: 79 -> 73.6 us; 1,024 rows 39.5 -> 38.6, 4,096 rows
+// 140 -> 131).  Non-temporal stores: 3.5 us less over 2,048 rows, 25 us more in a
+// 512-row decoder of four layers, where the next kernel reads the stored rows
+// from the caches: not used.
 #include <algorithm>
 #include <cmath>
 
@@ -41,16 +43,6 @@
 
 namespace sg {
 namespace {
-
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-
-// 16 bytes, with the non-temporal hint when kStream.
-template <bool kStream>
-__device__ __forceinline__ uint4 load16(const void* p) {
-  const u32x4* q = static_cast<const u32x4*>(p);
-  const u32x4 v = kStream ? __builtin_nontemporal_load(q) : *q;
-  return make_uint4(v[0], v[1], v[2], v[3]);
-}
 
 constexpr int kNormThreads = 256;
 
@@ -269,16 +261,11 @@ __global__ __launch_bounds__(kNormThreads) void qk_norm_rope_kernel(
 // out[r, i] = bf16(bf16(silu(gate[r, i])) * up[r, i]); gate = gu[r, :I],
 // up = gu[r, I:2I].  A workgroup takes 256 chunks of 8 elements of one row (parts =
 // workgroups per row), so that finding the row is one scalar division; two
-// chunks a thread measured 4 % slower.
-// kStream: non-temporal loads, for calls that move kStreamBytes or more.  Below,
-// what the projection before has just written is still in the 256 MB last-level
-// cache and the hint costs time; above, most of it is not, and the hint keeps
-// what is left for the next kernel.  The four stages of one layer (hidden 4096,
-// intermediate 12288) without / with the hint: 768 rows 32.3 / 35.6 us, 1,536
-// rows 51 / 58, 2,048 rows (151 MB here) 77 / 65.6, 4,096 rows 135 / 133.
-constexpr int64_t kStreamBytes = int64_t{128} << 20;
+// chunks a thread measured 4 % slower.  Plain loads: the non-temporal hint cost
+// 15 % on what the caches hold (2,048 x 12,288: 25.8 -> 29.7 us alone) and gave
+// nothing between the projections (up + SiLU + down 491 / 489 us at 2,048 rows,
+// 876 / 876 at 4,096) or in a layer's four calls on new inputs (75.4 / 77.4 us).
 constexpr int kSiluPart = 8 * 256;  // elements of a workgroup's part of a row
-template <bool kStream>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gu,
                                                        int64_t gu_stride, int inter,
                                                        uint16_t* __restrict__ out,
@@ -290,8 +277,8 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
     const uint32_t e = part * kSiluPart + 8 * threadIdx.x;
     if (e >= static_cast<uint32_t>(inter)) continue;
     const uint16_t* gr = gu + row * gu_stride + e;
-    const uint4 g = load16<kStream>(gr);
-    const uint4 u = load16<kStream>(gr + inter);
+    const uint4 g = *reinterpret_cast<const uint4*>(gr);
+    const uint4 u = *reinterpret_cast<const uint4*>(gr + inter);
     const uint32_t gv[4] = {g.x, g.y, g.z, g.w};
     const uint32_t uv[4] = {u.x, u.y, u.z, u.w};
     uint32_t o[4];
@@ -427,14 +414,10 @@ extern "C" int sg_silu_mul(const void* gate_up_dev, int64_t gate_up_row_stride,
   SG_REQUIRE(aligned16(gate_up_dev) && aligned16(out_dev), "tensors must be 16-byte aligned");
   const uint32_t parts = (static_cast<uint32_t>(intermediate) + kSiluPart - 1) / kSiluPart;
   const int64_t items = static_cast<int64_t>(num_rows) * parts;
-  auto go = [&](auto kernel) {
-    kernel<<<dim3(static_cast<unsigned>(std::min<int64_t>(items, 1 << 20))), dim3(256), 0,
-             static_cast<hipStream_t>(stream)>>>(
-        static_cast<const uint16_t*>(gate_up_dev), gate_up_row_stride, intermediate,
-        static_cast<uint16_t*>(out_dev), out_row_stride, parts, items);
-  };
-  const int64_t bytes = static_cast<int64_t>(num_rows) * intermediate * 6;  // two in, one out
-  bytes >= kStreamBytes ? go(silu_mul_kernel<true>) : go(silu_mul_kernel<false>);
+  silu_mul_kernel<<<dim3(static_cast<unsigned>(std::min<int64_t>(items, 1 << 20))), dim3(256), 0,
+                    static_cast<hipStream_t>(stream)>>>(
+      static_cast<const uint16_t*>(gate_up_dev), gate_up_row_stride, intermediate,
+      static_cast<uint16_t*>(out_dev), out_row_stride, parts, items);
   SG_LAUNCH_CHECK();
   return SG_OK;
 }
