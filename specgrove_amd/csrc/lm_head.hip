@@ -583,6 +583,13 @@ __global__ __launch_bounds__(kLmThreads, RowTile<R>::kBlocksPerCU) void lm_head_
 // most 63 empty rows.  A phase's MFMAs take 128 NB cycles beside 48 NB + 320
 // cycles of LDS traffic (the other group's fragment reads and the copies), so
 // a larger NB also spends fewer LDS cycles per product.
+//
+// Registers: all 256 of a wave (231 with the four-unit tile alone).  The five
+// tile sizes in one kernel spill 17 vector registers, all in the five-unit tile
+// (160 accumulators) and at nine places outside its main loops: the address
+// set-up, the last stages and the epilogue.  Scalar registers spill into vector
+// lanes (150 packed, 78 row-major, 10 before), read back outside the main loops
+// too.  A spill's memory access only makes a counted wait for copies stricter.
 constexpr int kPpThreads = 512;
 constexpr int kPpMaxUnits = 5;
 template <int NB>
@@ -674,16 +681,16 @@ __device__ __forceinline__ void pp_tile(const SgLmHeadArgs& a, unsigned char* sm
   // Fragments as in lm_head_kernel: lane l reads row l%16 of a 16-row block,
   // chunk l/16, at LDS chunk (l/16) ^ swz(l%16).
   const int lq = (lane & 15) * 64 + 16 * (g ^ (((lane & 15) >> 1) & 3));
-  const int a_base = wv * 8 * 1024;                // this wave's 128 token rows
-  const int b_base = kWBytes + wr * NB * 1024;     // this wave's hidden rows
+  const int a_base = wv * 8 * 1024;             // this wave's 128 token rows
+  const int b_base = kWBytes + wr * NB * 1024;  // this wave's hidden rows
 
-      // acc[tb][rb][i]: token 16 tb + 4 g + i of this wave's 128, row
-      // 16 rb + n of its 16 NB (lm_head_kernel's products and order).
-      floatx4 acc[8][NB];
+  // acc[tb][rb][i]: token 16 tb + 4 g + i of this wave's 128, row
+  // 16 rb + n of its 16 NB (lm_head_kernel's products and order).
+  floatx4 acc[8][NB];
 #pragma unroll
-      for (int tb = 0; tb < 8; ++tb)
+  for (int tb = 0; tb < 8; ++tb)
 #pragma unroll
-        for (int rb = 0; rb < NB; ++rb) acc[tb][rb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int rb = 0; rb < NB; ++rb) acc[tb][rb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // The main loop, once per group (G known at compile time, so each copy is
   // straight-line code: no branch chooses between product sites, which would

@@ -1230,7 +1230,9 @@ extern "C" int sg_tree_attn_plan(int32_t num_requests, const int32_t* row_offset
   // (hundredths of a microsecond on MI355X at 32q/8kv, D=128): a fixed part
   // (prologue latency, epilogue) plus a part per 32-key tile; a unit with at
   // most two q-groups (64 query vectors) streams two tiles per window and
-  // costs less per tile.
+  // costs less per tile.  Every row tile is charged all tree tiles of its
+  // request, here and in the splits above, though the kernel stops at the
+  // tile's last row.
   std::vector<int64_t> cost(units.size());
   for (size_t k = 0; k < units.size(); ++k) {
     const int rows = row_offset_host[units[k].req + 1] - row_offset_host[units[k].req];

@@ -337,8 +337,15 @@ def test_lm_head_row_tile_sizes_agree_bit_for_bit(device, oracle, vocab):
     _check_head(got, hidden, weight, rows, oracle)
 
 
+@pytest.fixture
+def dirty_status(monkeypatch):
+    """Status words that hold 7 before the call."""
+    monkeypatch.setattr(ops, "_new_status", lambda work, device:
+                        torch.full((1,), 7, dtype=torch.int32, device=device))
+
+
 @pytest.mark.parametrize("rows,bad", [(1, 0), (70, 69), (300, 299), (300, None)])
-def test_lm_head_writes_its_status(device, rows, bad):
+def test_lm_head_writes_its_status(device, dirty_status, rows, bad):
     """The call gives its status word its value, whatever the word held: the
     first workgroup of the row merge checks every index (256 threads, then a
     second round)."""
@@ -346,13 +353,12 @@ def test_lm_head_writes_its_status(device, rows, bad):
     index = torch.randint(0, 64, (rows,), device=device, dtype=torch.int32)
     if bad is not None:
         index[bad] = 64
-    junk = torch.full((1 << 12,), 7, dtype=torch.int32, device=device)
-    del junk  # the allocator hands its bytes to the next words
-    assert int(ops.lm_head(hidden, weight, index).status.item()) == (0 if bad is None else -1)
+    for w in (weight, ops.pack_lm_head(weight)):
+        assert int(ops.lm_head(hidden, w, index).status.item()) == (0 if bad is None else -1)
 
 
 @pytest.mark.parametrize("requests", [3, 65, 130])
-def test_projected_walk_writes_its_status(device, requests):
+def test_projected_walk_writes_its_status(device, dirty_status, requests):
     """One broken request anywhere (also past the 64 that one round of the
     status check reads) makes the call's status SG_EINVAL; none, SG_OK."""
     vocab, g = 300, torch.Generator(device=device).manual_seed(requests)
